@@ -204,14 +204,15 @@ enum : unsigned {
 
 // Separation runtime (dsp.hip), n_fft = 2048. chunk / audio [2][samples]; spectrum
 // [frames][1025][channel][re, im]; masks [2050][re, im][frames] (one stem); frames_buf
-// [frames][2][2048]; sums [2][total], weights [total].
+// [frames][2048][channel], 8-byte aligned; sums [2][total], weights [total].
 hipError_t launch_stft(const float* chunk, long samples, int hop, float* spectrum,
                        hipStream_t stream);
 hipError_t launch_istft_frames(const float* spectrum, const float* masks, int frames, int zero_dc,
                                float* frames_buf, hipStream_t stream);
 hipError_t launch_ola_accumulate(const float* frames_buf, int frames, int hop, long length,
                                  long start, long total, bool first, bool last, bool count_weight,
-                                 float* sums, float* weights, unsigned* flags, hipStream_t stream);
+                                 bool fresh, float* sums, float* weights, unsigned* flags,
+                                 hipStream_t stream);
 hipError_t launch_chunk_gather(const float* audio, long n, long start, long border,
                                long remaining, long samples, float* chunk, unsigned* flags,
                                hipStream_t stream);

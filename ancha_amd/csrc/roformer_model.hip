@@ -810,7 +810,7 @@ int ancha_hip_separate(ancha_hip_roformer* m, const float* audio, size_t samples
           e = ancha::launch_ola_accumulate(frames_buf, static_cast<int>(p.frames),
                                            static_cast<int>(m->hop), cs,
                                            static_cast<long>(start), length, first, last, s == 0,
-                                           sums + s * 2 * length, weights, flags, stream);
+                                           false, sums + s * 2 * length, weights, flags, stream);
         if (e != hipSuccess) return device_error(e);
       }
     }
@@ -870,14 +870,13 @@ int ancha_hip_istft(const float* spectrum, const float* masks, size_t frames, si
     return ancha::fail(ANCHA_HIP_INVALID, kWhere + "workspace too small or unaligned");
   float* frames_buf = static_cast<float*>(workspace);
   const long n = static_cast<long>(length);
-  hipError_t e = ancha::launch_zero(out, 2 * n, stream);
-  if (e == hipSuccess)
-    e = ancha::launch_istft_frames(spectrum, masks, static_cast<int>(frames), zero_dc ? 1 : 0,
-                                   frames_buf, stream);
-  // One chunk covering the whole output: unit fade weights (first and last).
+  hipError_t e = ancha::launch_istft_frames(spectrum, masks, static_cast<int>(frames),
+                                            zero_dc ? 1 : 0, frames_buf, stream);
+  // One chunk covering the whole output: unit fade weights (first and last), every sample written.
   if (e == hipSuccess)
     e = ancha::launch_ola_accumulate(frames_buf, static_cast<int>(frames), static_cast<int>(hop),
-                                     n, 0, n, true, true, false, out, nullptr, nullptr, stream);
+                                     n, 0, n, true, true, false, true, out, nullptr, nullptr,
+                                     stream);
   return ancha::hip_status(e, "ancha_hip_istft");
 }
 
@@ -889,7 +888,7 @@ int ancha_hip_istft(const float* spectrum, const float* masks, size_t frames, si
 
 namespace {
 
-// The windowed inverse frames [frames][2][2048] of one ancha_hip_istft_noalloc call. Every GPU
+// The windowed inverse frames [frames][2048][2] of one ancha_hip_istft_noalloc call. Every GPU
 // the library runs on holds its own copy (24 MiB) until the process ends. Host code uses only
 // the per-device address from hipGetSymbolAddress, never this name.
 constexpr size_t kIstftScratchFrames = 1536;

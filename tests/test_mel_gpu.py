@@ -73,6 +73,37 @@ def test_istft_round_trip_and_masks(gpu, n, hop):
         assert err < 1e-5 * max(np.abs(want).max(), 1.0)
 
 
+@pytest.mark.parametrize("frames,hop,offset", [(2, 441, 0), (3, 1024, 1), (4, 256, 0), (5, 441, 2),
+                                               (7, 300, 3), (33, 441, 1)])
+def test_istft_frame_groups_and_unaligned_spectrum(gpu, frames, hop, offset):
+    """Frame counts around the inverse kernel's groups of four frames, with the spectrum starting
+    `offset` floats past a 16-byte boundary: the result against the oracle (the same 1e-5 bound)
+    and, for an aligned copy of the spectrum, bit for bit. The STFT of the result's own length has
+    every frame reach past an end of the signal in the short cases (the reflected reads)."""
+    n = (frames - 1) * hop
+    m = W.normal((2050, 2, frames), 45, 1.0)
+    values = W.normal((frames * 4100 + 4,), 46, 1.0)
+    buf = torch.from_numpy(values).to(gpu)
+    spec = buf[offset:offset + frames * 4100].view(frames, 1025, 2, 2)
+    masks = torch.from_numpy(m).to(gpu)
+    y = S.istft(spec, masks, hop, n)
+    assert torch.equal(y, S.istft(spec.clone(), masks, hop, n))
+    sp = spec.cpu().numpy()
+    for c in range(2):
+        mc = (m[c::2, 0, :] + 1j * m[c::2, 1, :]).T
+        want = M.istft((sp[:, :, c, 0] + 1j * sp[:, :, c, 1]) * mc, n, 2048, hop)
+        err = np.abs(y[c].cpu().numpy() - want).max()
+        report(f"istft frames={frames} hop={hop} channel {c} max|diff|", err)
+        assert err < 1e-5 * max(np.abs(want).max(), 1.0)
+    if n > 1024:
+        x = W.audio(n, seed=47)
+        got = S.stft(torch.from_numpy(x).to(gpu), hop).cpu().numpy()
+        for c in range(2):
+            want = M.stft(x[c], 2048, hop)
+            assert np.abs(got[:, :, c, 0] + 1j * got[:, :, c, 1] - want).max() < (
+                1e-5 * np.abs(want).max())
+
+
 @pytest.mark.parametrize("depth", [1, 3])
 def test_forward_matches_oracle_tiny(gpu, depth):
     """Two stems, three overlapping bands, 101 frames (time kernel), 3 bands (band kernel).
