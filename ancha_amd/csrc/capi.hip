@@ -136,8 +136,8 @@ int run_attention(ancha::AttnParams& p, size_t groups, size_t tokens, size_t hea
 // offsets inside one 128-row tile.
 int run_linear(const float* x, size_t n, size_t k, size_t ldx, const float* w, size_t m,
                const float* bias, int gelu, const float* rope, size_t tokens, size_t width,
-               const float* residual, float* out, bool norm, hipStream_t stream,
-               const char* name) {
+               const float* residual, float* out, bool norm, void* workspace,
+               size_t workspace_bytes, hipStream_t stream, const char* name) {
   if (const int s = sticky()) return s;
   const std::string who(name);
   if (k == 0 || k % 8 != 0 || m == 0) return fail(ANCHA_HIP_UNSUPPORTED, who + ": k % 8 != 0 or empty");
@@ -173,7 +173,10 @@ int run_linear(const float* x, size_t n, size_t k, size_t ldx, const float* w, s
   const bool aligned = aligned16(x) && aligned16(w) && aligned16(out) &&
                        (!bias || aligned16(bias)) && (!residual || aligned16(residual)) &&
                        (!rope || aligned16(rope)) && ldx % 4 == 0 && m % 4 == 0;
-  const hipError_t e = ancha::launch_linear(p, aligned, stream);
+  const size_t need = workspace ? ancha::linear_wide_workspace(n, k, m) : 0;
+  const bool wide = aligned && need && workspace_bytes >= need && aligned16(workspace);
+  const hipError_t e = wide ? ancha::launch_linear_wide(p, workspace, stream)
+                            : ancha::launch_linear(p, aligned, stream);
   if (e != hipSuccess) return hip_fail(e, name);
   return ANCHA_HIP_OK;
 }
@@ -190,7 +193,23 @@ int ancha_hip_linear(const float* x, size_t n, size_t k, size_t ldx, const float
                      const float* bias, int gelu, const float* rope, size_t tokens, size_t width,
                      const float* residual, float* out, hipStream_t stream) {
   return run_linear(x, n, k, ldx, w, m, bias, gelu, rope, tokens, width, residual, out, false,
-                    stream, "ancha_hip_linear");
+                    nullptr, 0, stream, "ancha_hip_linear");
+}
+
+// Entry of the Python host mirror (fused.py): ancha_hip_linear (norm == 0) or ancha_hip_norm_linear
+// (norm != 0) with ancha_amd_linear_workspace(n, k, m) bytes of scratch, 16-byte aligned, for the
+// weight's fp16 fragments; with a null or short workspace, or where that returns 0, as those run.
+size_t ancha_amd_linear_workspace(size_t n, size_t k, size_t m) {
+  return ancha::linear_wide_workspace(n, k, m);
+}
+
+int ancha_amd_linear(const float* x, size_t n, size_t k, size_t ldx, const float* w, size_t m,
+                     const float* bias, int gelu, const float* rope, size_t tokens, size_t width,
+                     const float* residual, int norm, void* workspace, size_t workspace_bytes,
+                     float* out, hipStream_t stream) {
+  return run_linear(x, n, k, ldx, w, m, bias, gelu, rope, tokens, width, residual, out, norm != 0,
+                    workspace, workspace_bytes, stream, norm ? "ancha_hip_norm_linear"
+                                                             : "ancha_hip_linear");
 }
 
 int ancha_hip_norm_linear(const float* x, size_t n, size_t k, size_t ldx, const float* w,
@@ -198,7 +217,7 @@ int ancha_hip_norm_linear(const float* x, size_t n, size_t k, size_t ldx, const 
                           size_t tokens, size_t width, const float* residual, float* out,
                           hipStream_t stream) {
   return run_linear(x, n, k, ldx, w, m, bias, gelu, rope, tokens, width, residual, out, true,
-                    stream, "ancha_hip_norm_linear");
+                    nullptr, 0, stream, "ancha_hip_norm_linear");
 }
 
 int ancha_hip_swap_axes(const float* x, size_t batch, size_t a, size_t b, size_t dim, float* out,

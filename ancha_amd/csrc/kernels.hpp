@@ -66,6 +66,11 @@ struct LinearParams {
 // are multiples of 4.
 hipError_t launch_linear(const LinearParams& p, bool aligned, hipStream_t stream);
 
+// launch_linear for `aligned` calls with room for the fp16 weight fragments (linear_wide.hip):
+// linear_wide_workspace(n, k, m) bytes, 16-byte aligned; 0 where launch_linear is the path.
+size_t linear_wide_workspace(size_t n, size_t k, size_t m);
+hipError_t launch_linear_wide(const LinearParams& p, void* workspace, hipStream_t stream);
+
 // out[r] = x[r] / max(||x[r]||, 1e-12) * scale (scale [dim] or null): x [rows, dim] with row
 // stride ldx, out [rows, dim] contiguous; out may alias x when ldx == dim.
 struct NormParams {

@@ -161,9 +161,13 @@ def _linear(x: torch.Tensor, weight: torch.Tensor, epilogue: Epilogue,
         require(table, "rotary table", x.device)
     bias = None if epilogue.bias is None else epilogue.bias.contiguous()
     out = torch.empty((n, m), device=x.device, dtype=torch.float32)
-    fn = _native.lib().ancha_hip_norm_linear if norm else _native.lib().ancha_hip_linear
-    rc = fn(x.data_ptr(), n, k, x.stride(0), w.data_ptr(), m, _ptr(bias), int(epilogue.gelu),
-            _ptr(table), tokens, width, _ptr(residual), out.data_ptr(), _stream())
+    lib = _native.lib()
+    need = lib.ancha_amd_linear_workspace(n, k, m)
+    workspace = torch.empty(need, device=x.device, dtype=torch.uint8) if need else None
+    rc = lib.ancha_amd_linear(
+        x.data_ptr(), n, k, x.stride(0), w.data_ptr(), m, _ptr(bias), int(epilogue.gelu),
+        _ptr(table), tokens, width, _ptr(residual), int(norm), _ptr(workspace), need,
+        out.data_ptr(), _stream())
     return out if _native.check(rc) else None
 
 

@@ -321,3 +321,37 @@ def test_block_odd_head_count(gpu, tokens, heads):
     err = float(np.abs(got - want).max())
     print(f"block {heads} heads, T={tokens}: max|diff| {err:.3e}", flush=True)
     assert err < 2e-3
+
+
+# One case per tile form of the prepared-weight path and its edges: row blocks of 32 / 64 / 96 / 128
+# with a ragged last one, two and four k tiles in flight, one and several column groups, and the
+# resident form with its columns split and whole.
+@pytest.mark.parametrize("n,k,m,ldx", [
+    (1, 128, 128, 128), (33, 384, 1664, 388), (65, 640, 512, 640), (300, 1536, 384, 1536),
+    (2001, 512, 384, 516), (2600, 128, 1536, 128), (5000, 256, 1152, 256), (4003, 384, 1664, 384),
+    (2700, 512, 2048, 512), (12301, 256, 384, 256), (8200, 384, 512, 384), (16500, 128, 256, 128)])
+def test_prepared_weight_tiles(gpu, n, k, m, ldx):
+    rng = np.random.default_rng(5)
+    base = rng.standard_normal((n, ldx)).astype(np.float32)
+    x = base[:, :k]
+    x[n // 2] = 0.0
+    w = (0.05 * rng.standard_normal((k, m))).astype(np.float32)
+    b = rng.standard_normal(m).astype(np.float32)
+    r = rng.standard_normal((n, m)).astype(np.float32)
+    X, Wt, B, R = dev(base, gpu)[:, :k], dev(w, gpu), dev(b, gpu), dev(r, gpu)
+    rows = np.unique(np.concatenate([np.arange(min(n, 40)), np.arange(max(0, n - 140), n),
+                                     rng.integers(0, n, 60)]))
+    xs = np.ascontiguousarray(x[rows])
+    got = fused.linear(X, Wt, fused.Epilogue(bias=B, residual=R)).cpu().numpy()
+    assert np.isfinite(got).all()
+    check("bias + residual", got[rows], O.linear(xs, w, bias=b, residual=r[rows]), bound(xs, w))
+    xn = O.unit_norm(xs)
+    got = fused.norm_linear(X, Wt, fused.Epilogue(bias=B, gelu=True)).cpu().numpy()
+    check("norm + bias + GELU", got[rows], O.linear(xn, w, bias=b, gelu=True),
+          bound(xn, w, 1.13) + 1e-6)
+    # Rotary columns end inside the matrix; n tokens, so a row's token is the row.
+    width = m // 128 * 64 if m > 128 else 64
+    table = W.axis_rope_packed(W.rope_freqs(), n)
+    got = fused.linear(X, Wt, fused.Epilogue(rotary=(dev(table, gpu), width))).cpu().numpy()
+    want = O.linear(xs, w, rope=np.ascontiguousarray(table[:, rows]), tokens=len(rows), width=width)
+    check("rotary", got[rows], want, bound(xs, w, 1.42) + 1e-6)
