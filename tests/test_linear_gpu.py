@@ -124,6 +124,23 @@ def test_unit_norm(gpu, rows, dim, scaled):
     assert err < (2e-6 if scale is None else 5e-5)
 
 
+# Rows in registers: every count of vectors per lane, with the last one whole and ragged, aligned and
+# odd strides, a row count that ends inside a wave's rows, and the first length past the registers.
+@pytest.mark.parametrize("rows,dim,pad", [
+    (7, 4, 0), (5, 128, 0), (9, 132, 4), (33, 384, 0), (3, 388, 0), (6, 516, 12), (2, 1024, 0),
+    (3, 1028, 0), (1, 1, 0), (5, 65, 3), (9, 129, 0), (3, 400, 1), (7, 511, 0), (3, 640, 1),
+    (2, 767, 0), (5, 1023, 2), (3, 1025, 0)])
+def test_unit_norm_row_lengths(gpu, rows, dim, pad):
+    base = W.normal((rows, dim + pad), 43, 3.0)
+    x = np.ascontiguousarray(base[:, :dim])
+    scale = 1.0 + W.normal((dim,), 44, 0.1)
+    for s in (None, scale):
+        X = dev(base, gpu)[:, :dim]
+        got = fused.unit_norm(X, None if s is None else dev(s, gpu)).cpu().numpy()
+        # fp32 sums of up to 1028 squares: a relative error of some ulps on values of up to 1.4.
+        assert float(np.abs(got - O.unit_norm(x, s)).max()) < 2e-6
+
+
 def _block_weights(dim, heads, hidden, normalized=True):
     w, _ = C.layer_case() if (dim, heads, hidden) == (C.LAYER_DIM, C.LAYER_HEADS,
                                                       C.LAYER_HIDDEN) else (None, None)
@@ -193,6 +210,24 @@ def test_block_attention_core_at_layer_pair_shape(gpu, axis):
     err = float(np.abs(got - want).max())
     print(f"{axis} block output: max|diff| {err:.3e}", flush=True)
     assert err < 2e-3
+
+
+@pytest.mark.parametrize("dim,groups", [(384, (1, 150, 300, 1200)), (512, (1, 60, 150, 900))])
+def test_block_rows_do_not_depend_on_the_call_size(gpu, dim, groups):
+    """A sequence's rows are computed alike however many row blocks a call has: the projection's
+    columns split over six, three, two and one workgroups give the same bits."""
+    w = _block_weights(dim, 8, 4 * dim)
+    block = roformer.Transformer(w, gpu)
+    tokens = 33
+    table = roformer.axis_rope(w["freqs"], tokens, gpu)
+    x = dev(W.normal((groups[-1], tokens, dim), 71, 1.0), gpu)
+    whole = block(x, table)
+    want = O.transformer_forward(w, x[:1].cpu().numpy(), kernels=True, threads=8)
+    err = float(np.abs(whole[:1].cpu().numpy() - want).max())
+    print(f"block dim {dim}: max|diff| {err:.3e}", flush=True)
+    assert err < 2e-3
+    for g in groups[:-1]:
+        assert torch.equal(block(x[:g].contiguous(), table), whole[:g])
 
 
 def _oracle_pair(wt, wb, x):
