@@ -20,6 +20,16 @@
 // kPerm16 at load time. So x1 -> unit_norm -> fp16 and h -> fp16 go from accumulators to B
 // fragments in LDS with one 16-byte store per lane and no shuffles.
 //
+// Every transfer of rows is a set of contiguous pieces: the attended tile lands in LDS a kilobyte a
+// load, the residual and the two outputs pass through 4 KB of LDS of their wave as 128- or 64-byte
+// row pieces. A lane per row (16-byte pieces of 32 rows an access, as the accumulators and the
+// fragments have them) costs the address unit four times the cycles, and the weight loads of the
+// other workgroup wait behind it: 362 -> 336 us per call at 96 120 rows, dim 384 (341 -> 324 without
+// the fp16 output), 98 -> 90 us at 18 060 rows. The 16-byte stores have no scalar
+// offset: with one, the compiler leaves no wait state between the store and an instruction that
+// reuses its data registers, and on gfx950 the store's first dword then came out as the new value in
+// some lanes, now and then.
+//
 // Workgroup: 64 rows, 4 waves, one per feature quarter (and SIMD); two workgroups per CU, whose
 // phases drift apart, so one's GELU / norm VALU work runs beside the other's MFMAs. The out
 // accumulator (64 rows x dim) stays in registers from the residual load to the final store; the
@@ -39,6 +49,7 @@ constexpr int kRows = 64;         // rows per workgroup step
 constexpr int kChunk = 128;       // hidden units of one 32-unit block per wave (4 waves)
 constexpr int kWaves = 4;         // one per feature quarter (and per SIMD)
 constexpr int kFrag = 1024;       // bytes of one 32 x 16 fp16 fragment
+constexpr int kStage = 4096;      // bytes of one 32 x 32 fp32 tile on its way from or to whole rows
 // B fragments are read from LDS this many k steps ahead of their MFMAs (a scheduling barrier
 // per step keeps the reads there), so an MFMA never waits on a read issued just before it.
 constexpr int kBD = 2;
@@ -79,7 +90,9 @@ __global__ __launch_bounds__(kWaves * 64, 2) void block_tail_kernel(TailParams p
   constexpr int NB = NI <= 3 ? 2 : 1;
   constexpr int kCH = kChunk * NB;  // hidden units per chunk
   constexpr int kSC = kCH / 16;     // k steps of FF out per chunk
-  constexpr int kLds = (kRows * INNER * 2 > kX + kRows * kCH * 2) ? kRows * INNER * 2
+  // The attended tile with 4 KB per wave behind it, later X and H.
+  constexpr int kA = kRows * INNER * 2;
+  constexpr int kLds = kA + kWaves * kStage > kX + kRows * kCH * 2 ? kA + kWaves * kStage
                                                                    : kX + kRows * kCH * 2;
   static_assert(kLds <= 160 * 1024, "LDS");
   __shared__ __attribute__((aligned(16))) unsigned char lds[kLds];
@@ -87,13 +100,11 @@ __global__ __launch_bounds__(kWaves * 64, 2) void block_tail_kernel(TailParams p
   unsigned char* const H = lds + kX;    // hidden chunk: fragment (jb, s) at (jb * kSC + s) * 1 KB
   float* const red = reinterpret_cast<float*>(H);  // [4][128] row partials (aliases H)
 
-  const int tid = threadIdx.x, lane = tid & 63;
+  const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   constexpr int rh = 0;  // the workgroup's 64 rows are one pair of 32-row blocks
   const int fq = wave;
-  const int half = lane >> 5, col = lane & 31;
   const int hidden = p.hidden;
-  const unsigned lane16 = (unsigned)lane * 16;
 
   const rsrc_t wo = make_rsrc(p.wo, (unsigned)(DIM * INNER * 2));
   const rsrc_t w1 = make_rsrc(p.w1, (unsigned)(hidden * DIM * 2));
@@ -103,6 +114,11 @@ __global__ __launch_bounds__(kWaves * 64, 2) void block_tail_kernel(TailParams p
   const rsrc_t scr = make_rsrc(p.out_scale ? p.out_scale : p.b2, (unsigned)(DIM * 4));
 
   for (int blk = blockIdx.x; blk * kRows < p.rows; blk += gridDim.x) {
+    // Opaque per row block: the compiler cannot hold every lane address across the blocks.
+    int lane = tid & 63;
+    asm volatile("" : "+v"(lane));
+    const int half = lane >> 5, col = lane & 31;
+    const unsigned lane16 = (unsigned)lane * 16;
     const int row0 = blk * kRows;
     const int nrows = min(kRows, p.rows - row0);
     const rsrc_t att = make_rsrc(p.attended + (long)row0 * INNER, (unsigned)(nrows * INNER * 2));
@@ -111,32 +127,50 @@ __global__ __launch_bounds__(kWaves * 64, 2) void block_tail_kernel(TailParams p
     const rsrc_t xhr = make_rsrc(p.xh ? p.xh + (long)row0 * DIM : p.attended,
                                  p.xh ? (unsigned)(nrows * DIM * 2) : 0u);
 
-    // ---- the attended tile, straight into LDS as B fragments: fragment f = (jb, s) holds
-    // rows 32 jb + (l % 32), k 16 s + 8 (l / 32) .. + 7 in lane order.
-    for (int f = wave; f < 2 * S0; f += kWaves) {
-      const int jb = f / S0, s = f % S0;
-      const unsigned off = ((unsigned)(32 * jb + col) * INNER + 16 * s + 8 * half) * 2;
+    // ---- the attended tile, straight into LDS as rows of INNER halves: a load covers one
+    // contiguous kilobyte (one or four rows), 16-byte chunk c of row r landing at chunk
+    // c ^ (r & 15), so the 32 rows of a fragment read fall on 16 chunks.
+    constexpr int kChunks = INNER / 8;  // 16-byte chunks of a row
+    for (int f = wave; f < kA / kFrag; f += kWaves) {
+      const int r = (f * 64 + lane) / kChunks, c = (f * 64 + lane) % kChunks;
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          att, (__attribute__((address_space(3))) void*)(lds + f * kFrag), 16, off, 0, 0, 0);
+          att, (__attribute__((address_space(3))) void*)(lds + f * kFrag), 16,
+          (unsigned)(r * INNER * 2) + (unsigned)((c ^ (r & 15)) << 4), 0, 0, 0);
     }
     // ---- out accumulator = the residual x: lane holds row 32 (2 rh + j) + col, features
-    // fb + 8 q + 4 h .. + 3 (fb = 32 (fq NI + i)).
-    f32x16 acc[NI][2];
+    // fb + 8 q + 4 h .. + 3 (fb = 32 (fq NI + i)). Read as eight rows x 128 bytes a load and
+    // turned in this wave's staging area, 16-byte chunk c of row r at c ^ (r & 7).
+    unsigned char* const st = lds + kA + wave * kStage;
+    float4 xv[NI][2][4];
 #pragma unroll
     for (int i = 0; i < NI; i++)
 #pragma unroll
       for (int j = 0; j < 2; j++)
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
-          const float4 v = __builtin_bit_cast(
+        for (int k = 0; k < 4; k++)
+          xv[i][j][k] = __builtin_bit_cast(
               float4, __builtin_amdgcn_raw_buffer_load_b128(
-                          xr, ((unsigned)(32 * (2 * rh + j) + col) * DIM + 4 * half) * 4,
-                          (unsigned)(32 * (fq * NI + i) + 8 * q) * 4, 0));
+                          xr, ((unsigned)(32 * j + 8 * k + (lane >> 3)) * DIM + 4 * (lane & 7)) * 4,
+                          (unsigned)(32 * (fq * NI + i)) * 4, 0));
+    f32x16 acc[NI][2];
+#pragma unroll
+    for (int i = 0; i < NI; i++)
+#pragma unroll
+      for (int j = 0; j < 2; j++) {
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+          *reinterpret_cast<float4*>(st + (8 * k + (lane >> 3)) * 128 +
+                                     (((lane & 7) ^ (lane >> 3)) << 4)) = xv[i][j][k];
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+          const float4 v =
+              *reinterpret_cast<const float4*>(st + col * 128 + (((2 * q + half) ^ (col & 7)) << 4));
           acc[i][j][4 * q] = v.x;
           acc[i][j][4 * q + 1] = v.y;
           acc[i][j][4 * q + 2] = v.z;
           acc[i][j][4 * q + 3] = v.w;
         }
+      }
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
 
@@ -156,7 +190,8 @@ __global__ __launch_bounds__(kWaves * 64, 2) void block_tail_kernel(TailParams p
       auto load_b = [&](int s, u32x4 (&dst)[2]) {
 #pragma unroll
         for (int j = 0; j < 2; j++)
-          dst[j] = *reinterpret_cast<const u32x4*>(lds + ((2 * rh + j) * S0 + s) * kFrag + lane16);
+          dst[j] = *reinterpret_cast<const u32x4*>(
+              lds + (32 * (2 * rh + j) + col) * (INNER * 2) + (((2 * s + half) ^ (col & 15)) << 4));
       };
 #pragma unroll
       for (int s = 0; s < kBD; s++) load_b(s, b[s]);
@@ -314,21 +349,28 @@ __global__ __launch_bounds__(kWaves * 64, 2) void block_tail_kernel(TailParams p
     __syncthreads();  // H (the reduction buffer) is free again
 
     // ---- epilogue: + b2, optional output norm (and the next block's fp16 operand), stores.
+    {
+      float4 b[NI][4];  // all in flight together
 #pragma unroll
-    for (int i = 0; i < NI; i++)
+      for (int i = 0; i < NI; i++)
 #pragma unroll
-      for (int q = 0; q < 4; q++) {
-        const float4 b = __builtin_bit_cast(
-            float4, __builtin_amdgcn_raw_buffer_load_b128(
-                        b2r, 16 * half, (unsigned)(32 * (fq * NI + i) + 8 * q) * 4, 0));
+        for (int q = 0; q < 4; q++)
+          b[i][q] = __builtin_bit_cast(
+              float4, __builtin_amdgcn_raw_buffer_load_b128(
+                          b2r, 16 * half, (unsigned)(32 * (fq * NI + i) + 8 * q) * 4, 0));
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int j = 0; j < 2; j++) {
-          acc[i][j][4 * q] += b.x;
-          acc[i][j][4 * q + 1] += b.y;
-          acc[i][j][4 * q + 2] += b.z;
-          acc[i][j][4 * q + 3] += b.w;
-        }
-      }
+      for (int i = 0; i < NI; i++)
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+#pragma unroll
+          for (int j = 0; j < 2; j++) {
+            acc[i][j][4 * q] += b[i][q].x;
+            acc[i][j][4 * q + 1] += b[i][q].y;
+            acc[i][j][4 * q + 2] += b[i][q].z;
+            acc[i][j][4 * q + 3] += b[i][q].w;
+          }
+    }
     if (p.out_scale) {
       float part[2], tot[2];
 #pragma unroll
@@ -374,31 +416,45 @@ __global__ __launch_bounds__(kWaves * 64, 2) void block_tail_kernel(TailParams p
 #pragma unroll
       for (int j = 0; j < 2; j++) {
         const float inv = 1.0f / fmaxf(sqrtf(tot[j]), 1e-12f);
+        // Rows of 32 features (64 bytes) leave as 16 rows a store; chunk c of row r at c ^ (r & 3)
+        // of the staged tile.
 #pragma unroll
-        for (int i = 0; i < NI; i++)
+        for (int i = 0; i < NI; i++) {
 #pragma unroll
-          for (int q = 0; q < 4; q++) {
-            const u32x2 h = {pack_h2(acc[i][j][4 * q] * inv, acc[i][j][4 * q + 1] * inv),
-                             pack_h2(acc[i][j][4 * q + 2] * inv, acc[i][j][4 * q + 3] * inv)};
-            __builtin_amdgcn_raw_buffer_store_b64(
-                h, xhr, ((unsigned)(32 * (2 * rh + j) + col) * DIM + 4 * half) * 2,
-                (unsigned)(32 * (fq * NI + i) + 8 * q) * 2, 0);
+          for (int q = 0; q < 4; q++)
+            *reinterpret_cast<u32x2*>(st + col * 64 + ((q ^ (col & 3)) << 4) +
+                                      8 * half) =
+                u32x2{pack_h2(acc[i][j][4 * q] * inv, acc[i][j][4 * q + 1] * inv),
+                      pack_h2(acc[i][j][4 * q + 2] * inv, acc[i][j][4 * q + 3] * inv)};
+#pragma unroll
+          for (int k = 0; k < 2; k++) {
+            const int r = 16 * k + (lane >> 2), c = lane & 3;
+            __builtin_amdgcn_raw_buffer_store_b128(
+                *reinterpret_cast<const u32x4*>(st + r * 64 + ((c ^ (r & 3)) << 4)), xhr,
+                ((unsigned)(32 * (2 * rh + j) + r) * DIM + 32 * (fq * NI + i) + 8 * c) * 2, 0, 0);
           }
+        }
       }
     }
+    // Whole 128-byte row pieces through the staging area, eight rows a store.
 #pragma unroll
     for (int i = 0; i < NI; i++)
 #pragma unroll
-      for (int j = 0; j < 2; j++)
+      for (int j = 0; j < 2; j++) {
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
-          const float4 v = make_float4(acc[i][j][4 * q], acc[i][j][4 * q + 1],
-                                       acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]);
+        for (int q = 0; q < 4; q++)
+          *reinterpret_cast<u32x4*>(st + col * 128 + (((2 * q + half) ^ (col & 7)) << 4)) =
+              __builtin_bit_cast(u32x4, make_float4(acc[i][j][4 * q], acc[i][j][4 * q + 1],
+                                                    acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]));
+#pragma unroll
+        for (int k = 0; k < 4; k++)
           __builtin_amdgcn_raw_buffer_store_b128(
-              __builtin_bit_cast(u32x4, v), outr,
-              ((unsigned)(32 * (2 * rh + j) + col) * DIM + 4 * half) * 4,
-              (unsigned)(32 * (fq * NI + i) + 8 * q) * 4, 0);
-        }
+              *reinterpret_cast<const u32x4*>(st + (8 * k + (lane >> 3)) * 128 +
+                                              (((lane & 7) ^ (lane >> 3)) << 4)),
+              outr,
+              ((unsigned)(32 * (2 * rh + j) + 8 * k + (lane >> 3)) * DIM + 32 * (fq * NI + i) +
+               4 * (lane & 7)) * 4, 0, 0);
+      }
     __syncthreads();  // LDS is rewritten by the next row block's attended tile
   }
 }
