@@ -42,7 +42,7 @@ constexpr int kFrag = 1024;
 // TANH: the mask heads' hidden layer (bias + tanh on every column, no rotary table, p.batch
 // products of p.rows rows each).
 template <int SD, int NR, bool TANH = false>
-__global__ __launch_bounds__(kWaves * 64, 1) void qkv_kernel(QkvParams p) {
+__global__ __launch_bounds__(kWaves * 64, 1) void qkv_kernel(QkvParams p, int splits) {
   constexpr int kRows = 32 * NR;
   constexpr int kX = kRows * SD * 16 * 2;      // operand fragments
   // Per row: 16 chunks of (cos, sin) for two rotary pairs, chunk c at position c ^ (row & 15)
@@ -63,6 +63,9 @@ __global__ __launch_bounds__(kWaves * 64, 1) void qkv_kernel(QkvParams p) {
   const int half = lane >> 5, col = lane & 31;
   const unsigned lane16 = (unsigned)lane * 16;
   const int dim = SD * 16;
+  // This lane's 16 bytes of k step s: chunk 2 s + half of row `col` of a row tile, at
+  // (bo ^ 32 (s % 8)) + 256 (s / 8) (rows are whole 256-byte lines).
+  const int bo = col * dim * 2 + ((half ^ (col & 15)) << 4);
   // q, k, v and one gate column per head (all columns for TANH)
   const int used = TANH ? p.cols : 3 * p.width + p.width / 64;
   const int blocks = (used + 31) / 32;
@@ -110,8 +113,6 @@ __global__ __launch_bounds__(kWaves * 64, 1) void qkv_kernel(QkvParams p) {
     }
   };
 
-  // Pairs of this wave: wave + 8 n (n < mine); pair index % 4 = wave % 4 = its SIMD.
-  const int mine = pairs > wave ? (pairs - wave + kWaves - 1) / kWaves : 0;
   // k steps of weight fragments in flight (two fragments each): four at dims 384 (255 registers,
   // QKV 156 -> 150 us at 96 120 rows against two) and 512, two at dims 128 and 256.
   constexpr int PD = SD % 4 == 0 && SD > 16 ? 4 : 2;
@@ -119,13 +120,19 @@ __global__ __launch_bounds__(kWaves * 64, 1) void qkv_kernel(QkvParams p) {
 
   // Row blocks of each product (one product unless TANH).
   const int bpi = (p.rows + kRows - 1) / kRows;
-  const int total = TANH ? bpi * p.batch : bpi;
+  const int total = TANH ? bpi * p.batch : bpi * splits;
   // TANH: each product has weights of its own, so the row blocks of one product are kept on one
   // XCD (consecutive logical ids share an XCD) and its weights come into that XCD's L2 once.
   const int first = TANH ? xcd_remap(blockIdx.x, gridDim.x) : (int)blockIdx.x;
   for (int blk = first; blk < total; blk += gridDim.x) {
     const int item = TANH ? blk / bpi : 0;
-    const int row0 = (blk - item * bpi) * kRows;
+    // `splits` items share a row block's pairs; the last one has the odd block.
+    const int part = TANH ? 0 : blk % splits;
+    const int row0 = (TANH ? blk - item * bpi : blk / splits) * kRows;
+    const int p0 = TANH ? 0 : pairs * part / splits;
+    const int p1 = TANH ? pairs : pairs * (part + 1) / splits;
+    // Pairs of this wave: p0 + wave + 8 n (n < mine), the same count on every SIMD.
+    const int mine = p1 - p0 > wave ? (p1 - p0 - wave + kWaves - 1) / kWaves : 0;
     const int nrows = min(kRows, p.rows - row0);
     const rsrc_t xr = make_rsrc(p.xh + item * p.x_bstride + (long)row0 * dim,
                                 (unsigned)(nrows * dim * 2));
@@ -135,12 +142,14 @@ __global__ __launch_bounds__(kWaves * 64, 1) void qkv_kernel(QkvParams p) {
       wr = make_rsrc(p.w + item * p.w_bstride, (unsigned)(p.cols * dim * 2));
       br = make_rsrc(p.bias + item * p.b_bstride, (unsigned)(p.cols * 4));
     }
-    // Operand rows as B fragments: fragment (jb, s) = rows 32 jb + (l % 32), k 16 s + 8 (l / 32).
-    for (int f = wave; f < NR * SD; f += kWaves) {
-      const int jb = f / SD, s = f % SD;
+    // Operand rows as they lie in memory (a row block is contiguous, so a load covers one
+    // contiguous kilobyte), 16-byte chunk c of row r at chunk c ^ (r & 15): the 32 rows that a
+    // fragment read takes one chunk of fall on 16 chunks.
+    for (int f = wave; f < kX / kFrag; f += kWaves) {
+      const int r = (f * 64 + lane) / (2 * SD), c = (f * 64 + lane) % (2 * SD);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
           xr, (__attribute__((address_space(3))) void*)(lds + f * kFrag), 16,
-          ((unsigned)(32 * jb + col) * dim + 16 * s + 8 * half) * 2, 0, 0, 0);
+          (unsigned)(r * dim * 2) + (unsigned)((c ^ (r & 15)) << 4), 0, 0, 0);
     }
     // Key-table cos / sin of each row's token (the query tables are these times 1/8).
     for (int e = tid; e < (TANH ? 0 : kRows * 32); e += kWaves * 64) {
@@ -156,7 +165,7 @@ __global__ __launch_bounds__(kWaves * 64, 1) void qkv_kernel(QkvParams p) {
     // The A fragments of block 2 pr (x = 0) and 2 pr + 1 (x = 1) stream through the ring across
     // the wave's pairs; the last pair's last steps load the first steps of the odd block's tile
     // where the wave has one.
-    const bool tile_odd = odd && wave < NR;
+    const bool tile_odd = odd && wave < NR && part == splits - 1;
     u32x4 a[PD][2];
     if (mine > 0) {
 #pragma unroll
@@ -164,9 +173,9 @@ __global__ __launch_bounds__(kWaves * 64, 1) void qkv_kernel(QkvParams p) {
 #pragma unroll
         for (int x = 0; x < 2; x++)
           a[i][x] = __builtin_amdgcn_raw_buffer_load_b128(
-              wr, lane16, (unsigned)(((2 * wave + x) * SD + i) * kFrag), 0);
+              wr, lane16, (unsigned)(((2 * (p0 + wave) + x) * SD + i) * kFrag), 0);
       for (int n = 0; n < mine; n++) {
-        const int pr = wave + kWaves * n;
+        const int pr = p0 + wave + kWaves * n;
         // The operand fragments are the same for every pair; an opaque per-pair offset keeps
         // the compiler from hoisting all their LDS reads (NR * SD fragments) out of the loop.
         int opaque = 0;
@@ -201,7 +210,9 @@ __global__ __launch_bounds__(kWaves * 64, 1) void qkv_kernel(QkvParams p) {
           // pulling later steps' LDS reads forward.
 #pragma unroll
           for (int j = 0; j < NR; j++) {
-            const u32x4 bf = *reinterpret_cast<const u32x4*>(X + (j * SD + s) * kFrag + lane16);
+            const u32x4 bf =
+                *reinterpret_cast<const u32x4*>(X + j * (SD * kFrag) + (s >> 3) * 256 +
+                                                (bo ^ ((s & 7) << 5)));
 #pragma unroll
             for (int x = 0; x < 2; x++) acc[x][j] = mfma32(cur[x], bf, acc[x][j]);
           }
@@ -256,7 +267,9 @@ __global__ __launch_bounds__(kWaves * 64, 1) void qkv_kernel(QkvParams p) {
         if (s + PD < SD)
           a[s % PD][0] = __builtin_amdgcn_raw_buffer_load_b128(
               wr, lane16, (unsigned)((b * SD + s + PD) * kFrag), 0);
-        const u32x4 bf = *reinterpret_cast<const u32x4*>(lds + (j * SD + s) * kFrag + lane16);
+        const u32x4 bf =
+            *reinterpret_cast<const u32x4*>(lds + j * (SD * kFrag) + (s >> 3) * 256 +
+                                            (bo ^ ((s & 7) << 5)));
         acc = mfma32(cur, bf, acc);
       }
       u32x2 packed[4];
@@ -290,8 +303,20 @@ template <int SD, int NR = 4, bool TANH = false>
 hipError_t launch_t(const QkvParams& p, hipStream_t stream) {
   const int cus = device_cus();
   const int blocks = (p.rows + 32 * NR - 1) / (32 * NR) * (TANH ? p.batch : 1);
-  const int grid = blocks < cus ? blocks : cus;
-  hipLaunchKernelGGL((qkv_kernel<SD, NR, TANH>), dim3(grid), dim3(kWaves * 64), 0, stream, p);
+  // Fewer row blocks than CUs: the column pairs of one (24 and an odd block at eight heads, three
+  // per wave) split over two, three or six workgroups (one pair per SIMD) as long as that adds no
+  // round: 1024 rows 31.0 -> 15.0 us, 33 rows 28.8 -> 12.3, 4000 rows at dim 512 30.3 -> 17.6. Two
+  // rounds of thirds against one whole (142 row blocks) measured 38.9 against 36.9 us: not taken.
+  int splits = 1;
+  if (!TANH) {
+    const int pairs = (3 * p.width + p.width / 64 + 31) / 64;
+    splits = 6 * blocks <= cus ? 6 : 3 * blocks <= cus ? 3 : 2 * blocks <= cus ? 2 : 1;
+    while (splits > 1 && pairs < 4 * splits) splits--;
+  }
+  const int items = blocks * splits;
+  const int grid = items < cus ? items : cus;
+  hipLaunchKernelGGL((qkv_kernel<SD, NR, TANH>), dim3(grid), dim3(kWaves * 64), 0, stream, p,
+                     splits);
   return hipGetLastError();
 }
 
