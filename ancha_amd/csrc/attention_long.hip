@@ -33,8 +33,9 @@
 namespace ancha {
 namespace {
 
-constexpr int kWaves = 16;
-constexpr int kQueries = kWaves * 32;
+// Waves of a workgroup (NW): 16 on the persistent walk; 4 where 512-query passes leave the chip or
+// most of a workgroup idle (the launch below), one 128-query pass each.
+constexpr int kWalkWaves = 16;
 // Prefetch of the next pass's query rows, one chunk per K/V step: fp32 inputs in 8 chunks of 4
 // rows (each with its cos and sin table rows: 3 x 1 KB per wave), fp16 inputs in 4 chunks of 8
 // rows (1 KB per wave, loaded straight into place).
@@ -158,17 +159,22 @@ __device__ __forceinline__ void load_lds4(rsrc_t r, unsigned char* dst, unsigned
 // makes); otherwise their accesses are 4-byte ones (rows of an odd column count, e.g. a packed
 // projection with 1549 columns), with the same tiles and walk. TALIGNED: the same for the
 // rotary table.
-template <bool GATED, bool ROPE, bool XH, bool ALIGNED, bool TALIGNED = ALIGNED>
-__global__ __launch_bounds__(kWaves * 64, 1) void attention_long_kernel(AttnParams p, int qblocks,
-                                                                        int passes) {
+template <bool GATED, bool ROPE, bool XH, bool ALIGNED, bool TALIGNED, int NW>
+__global__ __launch_bounds__(NW * 64, NW == 16 ? 1 : XH || (!ROPE && ALIGNED) ? 3 : 2) void attention_long_kernel(AttnParams p,
+                                                                                  int qblocks,
+                                                                                  int passes) {
+  constexpr bool kWalk = NW == kWalkWaves;
+  constexpr int kQueries = NW * 32;
+  constexpr int kRowsPerThread = 16 / NW;  // K (and V) rows of a tile that a thread stages
+  constexpr int kRowStep = 4 * NW;         // and the distance between them
   // K tile: row = key (128 bytes of fp16 channels); V^T tile: row = channel (64 keys in
   // v_position order). Double buffered, the buffer index running on across passes.
   __shared__ __attribute__((aligned(16))) unsigned char lds_k[2][64 * 128];
   __shared__ __attribute__((aligned(16))) unsigned char lds_v[2][64 * 128];
   // Each wave's 32 queries of the next pass (fp16 rows), read into registers when it starts.
-  __shared__ __attribute__((aligned(16))) unsigned char lds_q[kWaves][32 * 128];
+  __shared__ __attribute__((aligned(16))) unsigned char lds_q[NW][32 * 128];
   // fp32 inputs: one prefetched chunk per wave (4 query rows, their cos rows, their sin rows).
-  __shared__ __attribute__((aligned(16))) unsigned char lds_raw[XH ? 1 : kWaves][XH ? 16 : 3072];
+  __shared__ __attribute__((aligned(16))) unsigned char lds_raw[XH || !kWalk ? 1 : NW][XH || !kWalk ? 16 : 3072];
   constexpr int kCh = kChunks<XH>;
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -223,8 +229,9 @@ __global__ __launch_bounds__(kWaves * 64, 1) void attention_long_kernel(AttnPara
   // and 2i + 1: V^T dwords pair them, and each lane writes two channels of its key pair (even
   // key: 4 sc, 4 sc + 1; odd key: 4 sc + 2, 4 sc + 3) after trading halves with its partner.
   // A write instruction's 32 lanes then cover both key pairs of the wave.
-  float4 kx = {}, kc = {}, ks = {}, vx = {};
-  u32x2 kh = {}, vh = {};
+  float4 kx[kRowsPerThread] = {}, kc[kRowsPerThread] = {}, ks[kRowsPerThread] = {},
+         vx[kRowsPerThread] = {};
+  u32x2 kh[kRowsPerThread] = {}, vh[kRowsPerThread] = {};
   // parts: 0 = K / V and the key table rows, 1 = K / V only, 2 = the table rows only.
   auto load_tile = [&](const unsigned char* kbase, const unsigned char* vbase, int key0,
                        int parts) {
@@ -234,12 +241,16 @@ __global__ __launch_bounds__(kWaves * 64, 1) void attention_long_kernel(AttnPara
     if (parts != 2) {
       const rsrc_t kr = make_rsrc(kbase + (long)key0 * ldk4, (rows - 1) * ldk4 + kRowBytes);
       const rsrc_t vr = make_rsrc(vbase + (long)key0 * ldv4, (rows - 1) * ldv4 + kRowBytes);
-      if constexpr (XH) {
-        kh = __builtin_amdgcn_raw_buffer_load_b64(kr, (unsigned)skey * ldk4 + sc * 8, 0, 0);
-        vh = __builtin_amdgcn_raw_buffer_load_b64(vr, (unsigned)vkey * ldv4 + sc * 8, 0, 0);
-      } else {
-        kx = bload4<ALIGNED>(kr, (unsigned)skey * ldk4 + sc * 16);
-        vx = bload4<ALIGNED>(vr, (unsigned)vkey * ldv4 + sc * 16);
+#pragma unroll
+      for (int i = 0; i < kRowsPerThread; i++) {
+        const unsigned kk = (unsigned)(skey + kRowStep * i), vk = (unsigned)(vkey + kRowStep * i);
+        if constexpr (XH) {
+          kh[i] = __builtin_amdgcn_raw_buffer_load_b64(kr, kk * ldk4 + sc * 8, 0, 0);
+          vh[i] = __builtin_amdgcn_raw_buffer_load_b64(vr, vk * ldv4 + sc * 8, 0, 0);
+        } else {
+          kx[i] = bload4<ALIGNED>(kr, kk * ldk4 + sc * 16);
+          vx[i] = bload4<ALIGNED>(vr, vk * ldv4 + sc * 16);
+        }
       }
     }
     if constexpr (ROPE && !XH) {
@@ -247,8 +258,11 @@ __global__ __launch_bounds__(kWaves * 64, 1) void attention_long_kernel(AttnPara
         // Key cos rows (table 2) and sign-folded sin rows (table 3) of this tile.
         const rsrc_t cr = make_rsrc(p.rope + (long)(2 * T + key0) * 64, rows * 256);
         const rsrc_t sr = make_rsrc(p.rope + (long)(3 * T + key0) * 64, rows * 256);
-        kc = bload4<TALIGNED>(cr, (unsigned)skey * 256 + sc * 16);
-        ks = bload4<TALIGNED>(sr, (unsigned)skey * 256 + sc * 16);
+#pragma unroll
+        for (int i = 0; i < kRowsPerThread; i++) {
+          kc[i] = bload4<TALIGNED>(cr, (unsigned)(skey + kRowStep * i) * 256 + sc * 16);
+          ks[i] = bload4<TALIGNED>(sr, (unsigned)(skey + kRowStep * i) * 256 + sc * 16);
+        }
       }
     }
   };
@@ -256,24 +270,29 @@ __global__ __launch_bounds__(kWaves * 64, 1) void attention_long_kernel(AttnPara
     const int skey = tid_o >> 4, sc = tid_o & 15;
     const int vkey = (skey & ~3) | ((skey & 1) << 1) | ((skey >> 1) & 1);
     const bool odd = (vkey & 1) != 0;
-    const int vch = 4 * sc + 2 * (int)odd, vpos = v_position(vkey & ~1);
-    u32x2 kw = kh, vw = vh;
-    if constexpr (!XH) {
-      float4 x = kx;
-      if constexpr (ROPE) x = rotate4(x, kc, ks);
-      kw = u32x2{pack_h2(x.x, x.y), pack_h2(x.z, x.w)};
-      vw = u32x2{pack_h2(vx.x, vx.y), pack_h2(vx.z, vx.w)};
+    const int vch = 4 * sc + 2 * (int)odd;
+#pragma unroll
+    for (int i = 0; i < kRowsPerThread; i++) {
+      const int vpos = v_position((vkey + kRowStep * i) & ~1);
+      u32x2 kw = kh[i], vw = vh[i];
+      if constexpr (!XH) {
+        float4 x = kx[i];
+        if constexpr (ROPE) x = rotate4(x, kc[i], ks[i]);
+        kw = u32x2{pack_h2(x.x, x.y), pack_h2(x.z, x.w)};
+        vw = u32x2{pack_h2(vx[i].x, vx[i].y), pack_h2(vx[i].z, vx[i].w)};
+      }
+      *reinterpret_cast<u32x2*>(lds_k[buf] + row_offset(skey + kRowStep * i, sc >> 1) +
+                                ((sc & 1) << 3)) = kw;
+      // Even key: (mine, partner's) of channels 4 sc, 4 sc + 1 (the partner sends its first
+      // dword); odd key: (partner's, mine) of 4 sc + 2, 4 sc + 3 (the partner sends its second).
+      const unsigned other = half_partner(odd ? vw[0] : vw[1], odd);
+      const unsigned lo = odd ? other : vw[0], hi = odd ? vw[1] : other;
+      unsigned char* V = lds_v[buf];
+      *reinterpret_cast<unsigned*>(V + v_offset(vch, vpos)) =
+          __builtin_amdgcn_perm(hi, lo, 0x05040100u);
+      *reinterpret_cast<unsigned*>(V + v_offset(vch + 1, vpos)) =
+          __builtin_amdgcn_perm(hi, lo, 0x07060302u);
     }
-    *reinterpret_cast<u32x2*>(lds_k[buf] + row_offset(skey, sc >> 1) + ((sc & 1) << 3)) = kw;
-    // Even key: (mine, partner's) of channels 4 sc, 4 sc + 1 (the partner sends its first
-    // dword); odd key: (partner's, mine) of 4 sc + 2, 4 sc + 3 (the partner sends its second).
-    const unsigned other = half_partner(odd ? vw[0] : vw[1], odd);
-    const unsigned lo = odd ? other : vw[0], hi = odd ? vw[1] : other;
-    unsigned char* V = lds_v[buf];
-    *reinterpret_cast<unsigned*>(V + v_offset(vch, vpos)) =
-        __builtin_amdgcn_perm(hi, lo, 0x05040100u);
-    *reinterpret_cast<unsigned*>(V + v_offset(vch + 1, vpos)) =
-        __builtin_amdgcn_perm(hi, lo, 0x07060302u);
   };
 
   // Query rows q0 .. q0 + 31 of (row0, head h); the buffer range ends at row T - 1, so rows
@@ -422,7 +441,7 @@ __global__ __launch_bounds__(kWaves * 64, 1) void attention_long_kernel(AttnPara
     const int q0n = qblkn * kQueries + wave * 32;
     const bool active_n = has_next && q0n < T;
     // The prefetch takes the last kCh K / V steps of the pass.
-    const bool prefetch = active_n && ntiles - 1 >= kCh;
+    const bool prefetch = kWalk && active_n && ntiles - 1 >= kCh;
     const int cstart = ntiles - 1 - kCh;
 
     // This wave's queries as B fragments of S^T = K.Q^T: fragment ds = query q0 + (l % 32),
@@ -539,10 +558,12 @@ __global__ __launch_bounds__(kWaves * 64, 1) void attention_long_kernel(AttnPara
           block(std::false_type{}, buf, 0, j * 64, std::false_type{});
       }
       load_tile(kbase, vbase, (j + 1) * 64, 2);
-      if (prefetch && c >= 0) issue_chunk(row0n, hn, q0n, c);
+      if constexpr (kWalk)
+        if (prefetch && c >= 0) issue_chunk(row0n, hn, q0n, c);
       if (active) block(std::false_type{}, buf, 1, j * 64, std::false_type{});
       __builtin_amdgcn_s_waitcnt(kWaitVmem);
-      if (prefetch && c >= 0) convert_chunk(c);
+      if constexpr (kWalk)
+        if (prefetch && c >= 0) convert_chunk(c);
       store_tile(buf ^ 1);
       __syncthreads();
       buf ^= 1;
@@ -602,14 +623,35 @@ __global__ __launch_bounds__(kWaves * 64, 1) void attention_long_kernel(AttnPara
 
 template <bool GATED, bool ROPE, bool XH, bool ALIGNED = true, bool TALIGNED = ALIGNED>
 hipError_t launch_t(const AttnParams& p, hipStream_t stream) {
-  const int qblocks = (p.tokens + kQueries - 1) / kQueries;
-  const int passes = p.groups * p.heads * qblocks;
+  const int problems = p.groups * p.heads;
+  const int qblocks = (p.tokens + 511) / 512;
+  const int passes = problems * qblocks;
+  const int cus = device_cus();
+  // 128-query passes on 4-wave workgroups (three a CU, two with fp32 rotary rows), none walking:
+  // up to 128 queries, where a 512-query workgroup has four waves busy of sixteen (200 x 100 x 8
+  // heads: 52.5 -> 31.8 us, with rotary 58.2 -> 39.0, 600 x 65 x 8 168 -> 70); with up to about one
+  // workgroup per CU (1 x 801 x 8 33.2 -> 19.3, 4 x 256 x 8 12.6 -> 10.0); and without rotary rows
+  // up to 384 tokens (200 x 256 x 8 120 -> 93, 60 x 301 x 8 40.2 -> 36.6) or five workgroups per CU
+  // (20 x 801 x 8 73 -> 60; 60 x 801 x 8 would be 161 against 147: more K / V traffic per query).
+  // With rotary rows every K row is rotated once per 128 queries: 129 - 256 tokens gain only from
+  // three workgroups per CU on (200 x 200 x 8 112 -> 105; 20 x 200 x 8 16.4 against 15.2), longer
+  // ones lose (60 x 400 x 8 79 against 62).
+  const int qb = (p.tokens + 127) / 128;
+  const long tiles = (long)problems * qb;
+  const bool heavy = ROPE && !XH;
+  const bool few = p.tokens <= 128 || tiles <= cus + cus / 8 ||
+                   (heavy ? p.tokens <= 256 && tiles >= 3l * cus
+                          : p.tokens <= 384 || tiles <= 5l * cus);
+  if (few && tiles < (1l << 23)) {  // 256 threads each: below HIP's 2^32 threads
+    hipLaunchKernelGGL((attention_long_kernel<GATED, ROPE, XH, ALIGNED, TALIGNED, 4>),
+                       dim3((unsigned)tiles), dim3(256), 0, stream, p, qb, (int)tiles);
+    return hipGetLastError();
+  }
   // One workgroup per CU walks the passes when there are more than two rounds of them; fewer
   // passes run one per workgroup (the walk would only lengthen the critical path).
-  const int cus = device_cus();
   const int grid = passes <= 2 * cus ? passes : cus;
-  hipLaunchKernelGGL((attention_long_kernel<GATED, ROPE, XH, ALIGNED, TALIGNED>), dim3(grid),
-                     dim3(kWaves * 64), 0, stream, p, qblocks, passes);
+  hipLaunchKernelGGL((attention_long_kernel<GATED, ROPE, XH, ALIGNED, TALIGNED, kWalkWaves>),
+                     dim3(grid), dim3(kWalkWaves * 64), 0, stream, p, qblocks, passes);
   return hipGetLastError();
 }
 

@@ -297,6 +297,30 @@ def test_tail_keys_are_attended_and_padding_is_masked(gpu, tokens):
     check(f"tail keys T={tokens}", got, expected)
 
 
+@pytest.mark.parametrize("groups,tokens,rope", [(41, 400, False), (33, 513, False), (22, 801, False),
+                                                (40, 130, True), (36, 256, True), (10, 801, True)])
+def test_small_and_walking_workgroups_agree(gpu, groups, tokens, rope):
+    """A call large enough for the 16-wave workgroups and its first groups alone, which take the
+    4-wave ones: both run the same arithmetic per 32 queries, so the same bits; oracle on a sample."""
+    q, k, v = (dev(W.normal((groups, tokens, 8, 64), s, 1.0), gpu) for s in (61, 62, 63))
+    table = W.axis_rope_packed(W.rope_freqs(), tokens) if rope else None
+    if not rope:
+        q = q / 8
+    t = dev(table, gpu) if rope else None
+    whole = fused.attention(q, k, v, rope=t)
+    few = 2 if tokens > 256 else 4
+    part = fused.attention(q[:few].contiguous(), k[:few].contiguous(), v[:few].contiguous(), rope=t)
+    assert torch.equal(part, whole[:few])
+    qn, kn, vn = (a[:1, :, :1].cpu().numpy() for a in (q, k, v))
+    if rope:
+        want = O.attention_op(np.ascontiguousarray(qn), np.ascontiguousarray(kn),
+                              np.ascontiguousarray(vn), rope=table)
+    else:
+        want = O.attention_op(np.ascontiguousarray(qn), np.ascontiguousarray(kn),
+                              np.ascontiguousarray(vn))
+    check(f"T={tokens}", whole[:1, :, :1].cpu().numpy(), want)
+
+
 @pytest.mark.parametrize("tokens", [96, 128, 130, 801, 1101])
 def test_time_attention_is_repeatable(gpu, tokens):
     """Three calls on the same inputs give identical bits, and all of them match the oracle.
