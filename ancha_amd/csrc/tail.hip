@@ -30,9 +30,9 @@
 // reuses its data registers, and on gfx950 the store's first dword then came out as the new value in
 // some lanes, now and then.
 //
-// Workgroup: 64 rows, 4 waves, one per feature quarter (and SIMD); two workgroups per CU, whose
+// Workgroup: 32 NJ rows (64; 32 in calls with few rows), 4 waves, one per feature quarter (and SIMD); two workgroups per CU, whose
 // phases drift apart, so one's GELU / norm VALU work runs beside the other's MFMAs. The out
-// accumulator (64 rows x dim) stays in registers from the residual load to the final store; the
+// accumulator (rows x dim) stays in registers from the residual load to the final store; the
 // hidden dimension runs in chunks of 256 units up to dim 384, 128 at dim 512 (per chunk: FF-in
 // for 64 or 32 hidden units per wave, GELU, the chunk's fp16 activation to LDS, then its FF-out
 // contribution).
@@ -45,7 +45,6 @@ namespace ancha {
 namespace {
 
 
-constexpr int kRows = 64;         // rows per workgroup step
 constexpr int kChunk = 128;       // hidden units of one 32-unit block per wave (4 waves)
 constexpr int kWaves = 4;         // one per feature quarter (and per SIMD)
 constexpr int kFrag = 1024;       // bytes of one 32 x 16 fp16 fragment
@@ -65,22 +64,23 @@ __device__ __forceinline__ u32x4 pack_frag(const f32x16& d, int sub, float s) {
 // Every wave calls it; it ends with the totals of this lane's rows in tot[].
 template <int NJ>
 __device__ __forceinline__ void row_totals(float* red, const float (&part)[NJ], float (&tot)[NJ],
-                                           int fq, int rh, int lane) {
+                                           int fq, int lane) {
   if (lane < 32)
 #pragma unroll
-    for (int j = 0; j < NJ; j++) red[fq * kRows + 32 * (2 * rh + j) + lane] = part[j];
+    for (int j = 0; j < NJ; j++) red[fq * (32 * NJ) + 32 * j + lane] = part[j];
   __syncthreads();
 #pragma unroll
   for (int j = 0; j < NJ; j++) {
-    const int row = 32 * (2 * rh + j) + (lane & 31);
-    tot[j] = red[row] + red[kRows + row] + red[2 * kRows + row] + red[3 * kRows + row];
+    const int row = 32 * j + (lane & 31);
+    tot[j] = red[row] + red[(32 * NJ) + row] + red[2 * (32 * NJ) + row] + red[3 * (32 * NJ) + row];
   }
   __syncthreads();
 }
 
 // DIM = 128 * NI features, INNER = heads * 64.
-template <int NI, int INNER>
+template <int NI, int INNER, int NJ>
 __global__ __launch_bounds__(kWaves * 64, 2) void block_tail_kernel(TailParams p) {
+  constexpr int kRows = 32 * NJ;  // rows per workgroup step
   constexpr int DIM = 128 * NI;
   constexpr int S0 = INNER / 16;   // k steps of the out projection
   constexpr int SD = DIM / 16;     // k steps of FF in
@@ -102,7 +102,6 @@ __global__ __launch_bounds__(kWaves * 64, 2) void block_tail_kernel(TailParams p
 
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  constexpr int rh = 0;  // the workgroup's 64 rows are one pair of 32-row blocks
   const int fq = wave;
   const int hidden = p.hidden;
 
@@ -137,26 +136,26 @@ __global__ __launch_bounds__(kWaves * 64, 2) void block_tail_kernel(TailParams p
           att, (__attribute__((address_space(3))) void*)(lds + f * kFrag), 16,
           (unsigned)(r * INNER * 2) + (unsigned)((c ^ (r & 15)) << 4), 0, 0, 0);
     }
-    // ---- out accumulator = the residual x: lane holds row 32 (2 rh + j) + col, features
+    // ---- out accumulator = the residual x: lane holds row 32 j + col, features
     // fb + 8 q + 4 h .. + 3 (fb = 32 (fq NI + i)). Read as eight rows x 128 bytes a load and
     // turned in this wave's staging area, 16-byte chunk c of row r at c ^ (r & 7).
     unsigned char* const st = lds + kA + wave * kStage;
-    float4 xv[NI][2][4];
+    float4 xv[NI][NJ][4];
 #pragma unroll
     for (int i = 0; i < NI; i++)
 #pragma unroll
-      for (int j = 0; j < 2; j++)
+      for (int j = 0; j < NJ; j++)
 #pragma unroll
         for (int k = 0; k < 4; k++)
           xv[i][j][k] = __builtin_bit_cast(
               float4, __builtin_amdgcn_raw_buffer_load_b128(
                           xr, ((unsigned)(32 * j + 8 * k + (lane >> 3)) * DIM + 4 * (lane & 7)) * 4,
                           (unsigned)(32 * (fq * NI + i)) * 4, 0));
-    f32x16 acc[NI][2];
+    f32x16 acc[NI][NJ];
 #pragma unroll
     for (int i = 0; i < NI; i++)
 #pragma unroll
-      for (int j = 0; j < 2; j++) {
+      for (int j = 0; j < NJ; j++) {
 #pragma unroll
         for (int k = 0; k < 4; k++)
           *reinterpret_cast<float4*>(st + (8 * k + (lane >> 3)) * 128 +
@@ -186,12 +185,12 @@ __global__ __launch_bounds__(kWaves * 64, 2) void block_tail_kernel(TailParams p
       };
 #pragma unroll
       for (int s = 0; s < PD; s++) load_a(s, a[s]);
-      u32x4 b[kBD + 1][2];
-      auto load_b = [&](int s, u32x4 (&dst)[2]) {
+      u32x4 b[kBD + 1][NJ];
+      auto load_b = [&](int s, u32x4 (&dst)[NJ]) {
 #pragma unroll
-        for (int j = 0; j < 2; j++)
+        for (int j = 0; j < NJ; j++)
           dst[j] = *reinterpret_cast<const u32x4*>(
-              lds + (32 * (2 * rh + j) + col) * (INNER * 2) + (((2 * s + half) ^ (col & 15)) << 4));
+              lds + (32 * j + col) * (INNER * 2) + (((2 * s + half) ^ (col & 15)) << 4));
       };
 #pragma unroll
       for (int s = 0; s < kBD; s++) load_b(s, b[s]);
@@ -206,16 +205,16 @@ __global__ __launch_bounds__(kWaves * 64, 2) void block_tail_kernel(TailParams p
 #pragma unroll
         for (int i = 0; i < NI; i++)
 #pragma unroll
-          for (int j = 0; j < 2; j++) acc[i][j] = mfma32(cur[i], b[s % (kBD + 1)][j], acc[i][j]);
+          for (int j = 0; j < NJ; j++) acc[i][j] = mfma32(cur[i], b[s % (kBD + 1)][j], acc[i][j]);
       }
     }
     __syncthreads();  // the attended tile is dead: X / H may be written
 
     // ---- xh1 = fp16(x1 / max(||x1||, 1e-12)) into X as FF-in B fragments.
     {
-      float part[2], tot[2];
+      float part[NJ], tot[NJ];
 #pragma unroll
-      for (int j = 0; j < 2; j++) {
+      for (int j = 0; j < NJ; j++) {
         float s = 0.f;
 #pragma unroll
         for (int i = 0; i < NI; i++)
@@ -223,16 +222,16 @@ __global__ __launch_bounds__(kWaves * 64, 2) void block_tail_kernel(TailParams p
           for (int r = 0; r < 16; r++) s += acc[i][j][r] * acc[i][j][r];
         part[j] = s + __shfl_xor(s, 32);
       }
-      row_totals<2>(red, part, tot, fq, rh, lane);
+      row_totals<NJ>(red, part, tot, fq, lane);
 #pragma unroll
-      for (int j = 0; j < 2; j++) {
+      for (int j = 0; j < NJ; j++) {
         const float inv = 1.0f / fmaxf(sqrtf(tot[j]), 1e-12f);
 #pragma unroll
         for (int i = 0; i < NI; i++)
 #pragma unroll
           for (int sub = 0; sub < 2; sub++) {
             const int s = 2 * (fq * NI + i) + sub;
-            *reinterpret_cast<u32x4*>(X + ((2 * rh + j) * SD + s) * kFrag + lane16) =
+            *reinterpret_cast<u32x4*>(X + (j * SD + s) * kFrag + lane16) =
                 pack_frag(acc[i][j], sub, inv);
           }
       }
@@ -244,7 +243,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void block_tail_kernel(TailParams p
       // FF in: this wave's hidden blocks NB fq + x (x < NB) of the chunk, units kCH c +
       // 32 (NB fq + x) + (8 q + 4 h + e), the accumulators starting at b1 (issued ahead of the
       // chunk's first weight fragments, which the first MFMA waits for anyway).
-      f32x16 hacc[NB][2];
+      f32x16 hacc[NB][NJ];
 #pragma unroll
       for (int x = 0; x < NB; x++)
 #pragma unroll
@@ -253,7 +252,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void block_tail_kernel(TailParams p
               float4, __builtin_amdgcn_raw_buffer_load_b128(
                           b1r, 16 * half, (unsigned)(kCH * c + 32 * (NB * fq + x) + 8 * q) * 4, 0));
 #pragma unroll
-          for (int j = 0; j < 2; j++) {
+          for (int j = 0; j < NJ; j++) {
             hacc[x][j][4 * q] = b.x;
             hacc[x][j][4 * q + 1] = b.y;
             hacc[x][j][4 * q + 2] = b.z;
@@ -272,11 +271,11 @@ __global__ __launch_bounds__(kWaves * 64, 2) void block_tail_kernel(TailParams p
         };
 #pragma unroll
         for (int s = 0; s < PD && s < SD; s++) load_a(s, a[s]);
-        u32x4 b[kBD + 1][2];
-        auto load_b = [&](int s, u32x4 (&dst)[2]) {
+        u32x4 b[kBD + 1][NJ];
+        auto load_b = [&](int s, u32x4 (&dst)[NJ]) {
 #pragma unroll
-          for (int j = 0; j < 2; j++)
-            dst[j] = *reinterpret_cast<const u32x4*>(X + ((2 * rh + j) * SD + s) * kFrag + lane16);
+          for (int j = 0; j < NJ; j++)
+            dst[j] = *reinterpret_cast<const u32x4*>(X + (j * SD + s) * kFrag + lane16);
         };
 #pragma unroll
         for (int s = 0; s < kBD; s++) load_b(s, b[s]);
@@ -291,7 +290,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void block_tail_kernel(TailParams p
 #pragma unroll
           for (int x = 0; x < NB; x++)
 #pragma unroll
-            for (int j = 0; j < 2; j++)
+            for (int j = 0; j < NJ; j++)
               hacc[x][j] = mfma32(cur[x], b[s % (kBD + 1)][j], hacc[x][j]);
         }
       }
@@ -300,13 +299,13 @@ __global__ __launch_bounds__(kWaves * 64, 2) void block_tail_kernel(TailParams p
 #pragma unroll
       for (int x = 0; x < NB; x++)
 #pragma unroll
-        for (int j = 0; j < 2; j++) {
+        for (int j = 0; j < NJ; j++) {
           f32x16 g;
 #pragma unroll
           for (int r = 0; r < 16; r++) g[r] = gemm::gelu_fast(hacc[x][j][r]);
 #pragma unroll
           for (int sub = 0; sub < 2; sub++)
-            *reinterpret_cast<u32x4*>(H + ((2 * rh + j) * kSC + 2 * (NB * fq + x) + sub) * kFrag +
+            *reinterpret_cast<u32x4*>(H + (j * kSC + 2 * (NB * fq + x) + sub) * kFrag +
                                       lane16) = pack_frag(g, sub, 1.0f);
         }
       __syncthreads();
@@ -323,11 +322,11 @@ __global__ __launch_bounds__(kWaves * 64, 2) void block_tail_kernel(TailParams p
         };
 #pragma unroll
         for (int s = 0; s < PD; s++) load_a(s, a[s]);
-        u32x4 b[kBD + 1][2];
-        auto load_b = [&](int s, u32x4 (&dst)[2]) {
+        u32x4 b[kBD + 1][NJ];
+        auto load_b = [&](int s, u32x4 (&dst)[NJ]) {
 #pragma unroll
-          for (int j = 0; j < 2; j++)
-            dst[j] = *reinterpret_cast<const u32x4*>(H + ((2 * rh + j) * kSC + s) * kFrag + lane16);
+          for (int j = 0; j < NJ; j++)
+            dst[j] = *reinterpret_cast<const u32x4*>(H + (j * kSC + s) * kFrag + lane16);
         };
 #pragma unroll
         for (int s = 0; s < kBD; s++) load_b(s, b[s]);
@@ -342,7 +341,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void block_tail_kernel(TailParams p
 #pragma unroll
           for (int i = 0; i < NI; i++)
 #pragma unroll
-            for (int j = 0; j < 2; j++) acc[i][j] = mfma32(cur[i], b[s % (kBD + 1)][j], acc[i][j]);
+            for (int j = 0; j < NJ; j++) acc[i][j] = mfma32(cur[i], b[s % (kBD + 1)][j], acc[i][j]);
         }
       }
     }
@@ -364,7 +363,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void block_tail_kernel(TailParams p
 #pragma unroll
         for (int q = 0; q < 4; q++)
 #pragma unroll
-          for (int j = 0; j < 2; j++) {
+          for (int j = 0; j < NJ; j++) {
             acc[i][j][4 * q] += b[i][q].x;
             acc[i][j][4 * q + 1] += b[i][q].y;
             acc[i][j][4 * q + 2] += b[i][q].z;
@@ -372,9 +371,9 @@ __global__ __launch_bounds__(kWaves * 64, 2) void block_tail_kernel(TailParams p
           }
     }
     if (p.out_scale) {
-      float part[2], tot[2];
+      float part[NJ], tot[NJ];
 #pragma unroll
-      for (int j = 0; j < 2; j++) {
+      for (int j = 0; j < NJ; j++) {
         float s = 0.f;
 #pragma unroll
         for (int i = 0; i < NI; i++)
@@ -382,9 +381,9 @@ __global__ __launch_bounds__(kWaves * 64, 2) void block_tail_kernel(TailParams p
           for (int r = 0; r < 16; r++) s += acc[i][j][r] * acc[i][j][r];
         part[j] = s + __shfl_xor(s, 32);
       }
-      row_totals<2>(red, part, tot, fq, rh, lane);
+      row_totals<NJ>(red, part, tot, fq, lane);
 #pragma unroll
-      for (int j = 0; j < 2; j++) {
+      for (int j = 0; j < NJ; j++) {
         const float inv = 1.0f / fmaxf(sqrtf(tot[j]), 1e-12f);
 #pragma unroll
         for (int i = 0; i < NI; i++)
@@ -402,9 +401,9 @@ __global__ __launch_bounds__(kWaves * 64, 2) void block_tail_kernel(TailParams p
     }
     if (p.xh) {
       // The next block's fp16 operand, fp16(unit_norm(y)) (y after the output norm, if any).
-      float part[2], tot[2];
+      float part[NJ], tot[NJ];
 #pragma unroll
-      for (int j = 0; j < 2; j++) {
+      for (int j = 0; j < NJ; j++) {
         float s = 0.f;
 #pragma unroll
         for (int i = 0; i < NI; i++)
@@ -412,9 +411,9 @@ __global__ __launch_bounds__(kWaves * 64, 2) void block_tail_kernel(TailParams p
           for (int r = 0; r < 16; r++) s += acc[i][j][r] * acc[i][j][r];
         part[j] = s + __shfl_xor(s, 32);
       }
-      row_totals<2>(red, part, tot, fq, rh, lane);
+      row_totals<NJ>(red, part, tot, fq, lane);
 #pragma unroll
-      for (int j = 0; j < 2; j++) {
+      for (int j = 0; j < NJ; j++) {
         const float inv = 1.0f / fmaxf(sqrtf(tot[j]), 1e-12f);
         // Rows of 32 features (64 bytes) leave as 16 rows a store; chunk c of row r at c ^ (r & 3)
         // of the staged tile.
@@ -431,7 +430,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void block_tail_kernel(TailParams p
             const int r = 16 * k + (lane >> 2), c = lane & 3;
             __builtin_amdgcn_raw_buffer_store_b128(
                 *reinterpret_cast<const u32x4*>(st + r * 64 + ((c ^ (r & 3)) << 4)), xhr,
-                ((unsigned)(32 * (2 * rh + j) + r) * DIM + 32 * (fq * NI + i) + 8 * c) * 2, 0, 0);
+                ((unsigned)(32 * j + r) * DIM + 32 * (fq * NI + i) + 8 * c) * 2, 0, 0);
           }
         }
       }
@@ -440,7 +439,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void block_tail_kernel(TailParams p
 #pragma unroll
     for (int i = 0; i < NI; i++)
 #pragma unroll
-      for (int j = 0; j < 2; j++) {
+      for (int j = 0; j < NJ; j++) {
 #pragma unroll
         for (int q = 0; q < 4; q++)
           *reinterpret_cast<u32x4*>(st + col * 128 + (((2 * q + half) ^ (col & 7)) << 4)) =
@@ -452,7 +451,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void block_tail_kernel(TailParams p
               *reinterpret_cast<const u32x4*>(st + (8 * k + (lane >> 3)) * 128 +
                                               (((lane & 7) ^ (lane >> 3)) << 4)),
               outr,
-              ((unsigned)(32 * (2 * rh + j) + 8 * k + (lane >> 3)) * DIM + 32 * (fq * NI + i) +
+              ((unsigned)(32 * j + 8 * k + (lane >> 3)) * DIM + 32 * (fq * NI + i) +
                4 * (lane & 7)) * 4, 0, 0);
       }
     __syncthreads();  // LDS is rewritten by the next row block's attended tile
@@ -460,8 +459,20 @@ __global__ __launch_bounds__(kWaves * 64, 2) void block_tail_kernel(TailParams p
 }
 
 template <int NI, int INNER>
-hipError_t launch_t(const TailParams& p, int grid, hipStream_t stream) {
-  hipLaunchKernelGGL((block_tail_kernel<NI, INNER>), dim3(grid), dim3(kWaves * 64), 0, stream, p);
+hipError_t launch_t(const TailParams& p, hipStream_t stream) {
+  const int cus = device_cus();
+  // 32-row blocks while they leave no CU with two: half the MFMAs behind the same weight stream
+  // (33 rows 42.8 -> 32.6 us, 4000 rows 48.7 -> 41.4, 8000 52.3 -> 49.2; at 10 240 rows, with two on
+  // some CUs, 65.8 against 55.8).
+  if ((p.rows + 31) / 32 <= cus) {
+    const int blocks = (p.rows + 31) / 32;
+    hipLaunchKernelGGL((block_tail_kernel<NI, INNER, 1>), dim3(blocks), dim3(kWaves * 64), 0, stream,
+                       p);
+    return hipGetLastError();
+  }
+  const int blocks = (p.rows + 63) / 64;  // two workgroups per CU
+  hipLaunchKernelGGL((block_tail_kernel<NI, INNER, 2>), dim3(blocks < 2 * cus ? blocks : 2 * cus),
+                     dim3(kWaves * 64), 0, stream, p);
   return hipGetLastError();
 }
 
@@ -477,23 +488,20 @@ bool block_tail_supported(int dim, int inner, int hidden) {
 hipError_t launch_block_tail(const TailParams& p, hipStream_t stream) {
   if (!block_tail_supported(p.dim, p.inner, p.hidden)) return hipErrorInvalidValue;
   if (p.rows <= 0) return hipSuccess;
-  const int cus = device_cus();
-  const int blocks = (p.rows + kRows - 1) / kRows;
-  const int grid = blocks < 2 * cus ? blocks : 2 * cus;  // two workgroups per CU
   const int ni = p.dim / 128;
   if (p.inner == 512) {
     switch (ni) {
-      case 1: return launch_t<1, 512>(p, grid, stream);
-      case 2: return launch_t<2, 512>(p, grid, stream);
-      case 3: return launch_t<3, 512>(p, grid, stream);
-      default: return launch_t<4, 512>(p, grid, stream);
+      case 1: return launch_t<1, 512>(p, stream);
+      case 2: return launch_t<2, 512>(p, stream);
+      case 3: return launch_t<3, 512>(p, stream);
+      default: return launch_t<4, 512>(p, stream);
     }
   }
   switch (ni) {
-    case 1: return launch_t<1, 128>(p, grid, stream);
-    case 2: return launch_t<2, 128>(p, grid, stream);
-    case 3: return launch_t<3, 128>(p, grid, stream);
-    default: return launch_t<4, 128>(p, grid, stream);
+    case 1: return launch_t<1, 128>(p, stream);
+    case 2: return launch_t<2, 128>(p, stream);
+    case 3: return launch_t<3, 128>(p, stream);
+    default: return launch_t<4, 128>(p, stream);
   }
 }
 
