@@ -20,6 +20,10 @@ def _index(device: torch.device) -> int:
 def require(t: torch.Tensor, name: str, device: torch.device,
             shape: Optional[Sequence[int]] = None, dtype: torch.dtype = torch.float32) -> None:
     """Raise ValueError unless ``t`` is a ``dtype`` tensor on ``device`` (and of ``shape``)."""
+    # All in order (an indexed device): two comparisons. The rest names what is not.
+    if (isinstance(t, torch.Tensor) and t.dtype == dtype and t.is_cuda and t.device == device
+            and (shape is None or t.shape == torch.Size(shape))):
+        return
     if not isinstance(t, torch.Tensor):
         raise ValueError(f"{name} must be a torch tensor")
     if t.dtype != dtype:

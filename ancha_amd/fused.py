@@ -26,8 +26,14 @@ def available() -> bool:
     return bool(_native.lib().ancha_hip_available())
 
 
+def _usable() -> bool:
+    """available() for a caller that already holds a GPU tensor."""
+    return bool(_native.lib().ancha_hip_available())
+
+
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    """torch.cuda.current_stream().cuda_stream without the Stream object."""
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
@@ -41,6 +47,9 @@ def _rows(t: torch.Tensor) -> tuple[torch.Tensor, int]:
     if t.dtype != torch.float32:
         raise ValueError("fused ops take float32 tensors")
     g, tok = t.shape[0], t.shape[1]
+    if t.is_contiguous():
+        # Dense as it is; callers use only its address and this stride.
+        return t, t.shape[2] * t.shape[3] if t.dim() == 4 else t.shape[2]
     try:
         flat = t.view(g, tok, -1)
     except RuntimeError:
@@ -68,15 +77,14 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     query table carries 1/sqrt(64))."""
     if q.dim() != 4 or q.shape[3] != ATTENTION_HEAD_DIM or k.shape != q.shape or v.shape != q.shape:
         return None
-    if not q.is_cuda or not available():
+    if not q.is_cuda or not _usable():
         return None
     for name, t in (("q", q), ("k", k), ("v", v)):
         require(t, name, q.device)
     groups, tokens, heads, _ = q.shape
     (qf, ldq), (kf, ldk), (vf, ldv) = (_rows(t) for t in (q, k, v))
     table = _table(rope, tokens, q.device)
-    out = torch.empty((groups, tokens, heads, ATTENTION_HEAD_DIM), device=q.device,
-                      dtype=torch.float32)
+    out = q.new_empty((groups, tokens, heads, ATTENTION_HEAD_DIM))
     rc = _native.lib().ancha_hip_attention(
         qf.data_ptr(), kf.data_ptr(), vf.data_ptr(), groups, tokens, heads, ldq, ldk, ldv,
         _ptr(table), out.data_ptr(), _stream())
@@ -90,7 +98,7 @@ def gated_attention(packed: torch.Tensor, heads: int,
     softmax(q.k^T).v * sigmoid(gate) as [groups, tokens, heads, 64], or None."""
     if packed.dim() != 3 or packed.shape[2] < heads * (3 * ATTENTION_HEAD_DIM + 1):
         return None
-    if not packed.is_cuda or not available():
+    if not packed.is_cuda or not _usable():
         return None
     require(packed, "packed", packed.device)
     groups, tokens, columns = packed.shape
@@ -98,8 +106,7 @@ def gated_attention(packed: torch.Tensor, heads: int,
     if ld != columns:
         flat, ld = flat.contiguous(), columns
     table = _table(rope, tokens, packed.device)
-    out = torch.empty((groups, tokens, heads, ATTENTION_HEAD_DIM), device=packed.device,
-                      dtype=torch.float32)
+    out = packed.new_empty((groups, tokens, heads, ATTENTION_HEAD_DIM))
     rc = _native.lib().ancha_hip_gated_attention(
         flat.data_ptr(), groups, tokens, columns, heads, _ptr(table), out.data_ptr(), _stream())
     return out if _native.check(rc) else None
@@ -151,7 +158,7 @@ def _linear(x: torch.Tensor, weight: torch.Tensor, epilogue: Epilogue,
         if tuple(residual.shape) != (n, m):
             return None
         residual = residual.contiguous()
-    if not x.is_cuda or not available():
+    if not x.is_cuda or not _usable():
         return None
     x = _matrix(x, "x", x.device)
     w = _matrix(weight, "weight", x.device).contiguous()
@@ -160,7 +167,7 @@ def _linear(x: torch.Tensor, weight: torch.Tensor, epilogue: Epilogue,
     if table is not None:
         require(table, "rotary table", x.device)
     bias = None if epilogue.bias is None else epilogue.bias.contiguous()
-    out = torch.empty((n, m), device=x.device, dtype=torch.float32)
+    out = x.new_empty((n, m))
     lib = _native.lib()
     need = lib.ancha_amd_linear_workspace(n, k, m)
     workspace = torch.empty(need, device=x.device, dtype=torch.uint8) if need else None
@@ -193,12 +200,12 @@ def unit_norm(x: torch.Tensor, scale: Optional[torch.Tensor] = None) -> torch.Te
         raise ValueError("unit_norm takes a float32 CUDA tensor")
     dim = x.shape[-1]
     require_optional(scale, "scale", x.device, (dim,))
-    if not available():
+    if not _usable():
         raise RuntimeError("the gfx950 kernels cannot run on this device")
-    flat = x.reshape(-1, dim)
+    flat = x if x.dim() == 2 else x.reshape(-1, dim)
     if flat.stride(1) != 1:
         flat = flat.contiguous()
-    out = torch.empty(x.shape, device=x.device, dtype=torch.float32)
+    out = x.new_empty(x.shape)
     s = None if scale is None else scale.contiguous()
     rc = _native.lib().ancha_hip_unit_norm(flat.data_ptr(), flat.shape[0], dim, flat.stride(0),
                                            _ptr(s), out.data_ptr(), _stream())
