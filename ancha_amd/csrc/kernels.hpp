@@ -128,7 +128,7 @@ struct Gemm16Params {
 
 hipError_t launch_gemm16(const Gemm16Params& p, hipStream_t stream);
 
-// Fused tail of the RoFormer block (tail.hip), 128 rows per workgroup step:
+// Fused tail of the RoFormer block (tail.hip):
 //   x1 = x + attended . W_out; h = fp16(GELU(fp16(unit_norm(x1)) . W1' + b1));
 //   out = x1 + h . W2 + b2; with out_scale: out = unit_norm(out) * out_scale and, with xh,
 //   xh = fp16(unit_norm(out)).

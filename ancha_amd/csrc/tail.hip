@@ -25,14 +25,14 @@
 // row pieces. A lane per row (16-byte pieces of 32 rows an access, as the accumulators and the
 // fragments have them) costs the address unit four times the cycles, and the weight loads of the
 // other workgroup wait behind it: 362 -> 336 us per call at 96 120 rows, dim 384 (341 -> 324 without
-// the fp16 output), 98 -> 90 us at 18 060 rows. The 16-byte stores have no scalar
-// offset: with one, the compiler leaves no wait state between the store and an instruction that
-// reuses its data registers, and on gfx950 the store's first dword then came out as the new value in
-// some lanes, now and then.
+// the fp16 output), 98 -> 90 us at 18 060 rows. The 16-byte stores have no scalar offset: with one,
+// the compiler leaves no wait state between the store and an instruction that reuses its data
+// registers, and on gfx950 the store's first dword then came out as the new value in some lanes, now
+// and then.
 //
-// Workgroup: 32 NJ rows (64; 32 in calls with few rows), 4 waves, one per feature quarter (and SIMD); two workgroups per CU, whose
-// phases drift apart, so one's GELU / norm VALU work runs beside the other's MFMAs. The out
-// accumulator (rows x dim) stays in registers from the residual load to the final store; the
+// Workgroup: 32 NJ rows (64; 32 in calls with few rows), 4 waves, one per feature quarter (and
+// SIMD); two workgroups per CU, whose phases drift apart, so one's GELU / norm VALU work runs beside
+// the other's MFMAs. The out accumulator (rows x dim) stays in registers from the residual load to the final store; the
 // hidden dimension runs in chunks of 256 units up to dim 384, 128 at dim 512 (per chunk: FF-in
 // for 64 or 32 hidden units per wave, GELU, the chunk's fp16 activation to LDS, then its FF-out
 // contribution).
@@ -43,7 +43,6 @@
 
 namespace ancha {
 namespace {
-
 
 constexpr int kChunk = 128;       // hidden units of one 32-unit block per wave (4 waves)
 constexpr int kWaves = 4;         // one per feature quarter (and per SIMD)
@@ -81,6 +80,9 @@ __device__ __forceinline__ void row_totals(float* red, const float (&part)[NJ], 
 template <int NI, int INNER, int NJ>
 __global__ __launch_bounds__(kWaves * 64, 2) void block_tail_kernel(TailParams p) {
   constexpr int kRows = 32 * NJ;  // rows per workgroup step
+  // k steps of weight fragments in flight, out projection / FF out and FF in (twice to three times
+  // as many with one row block: parity at dim 384, 69 against 66 us at dim 512).
+  constexpr int kPdOut = NI > 3 ? 2 : 4, kPdIn = NI > 3 ? 8 : 4;
   constexpr int DIM = 128 * NI;
   constexpr int S0 = INNER / 16;   // k steps of the out projection
   constexpr int SD = DIM / 16;     // k steps of FF in
@@ -175,7 +177,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void block_tail_kernel(TailParams p
 
     // ---- out projection: acc += W_out^T . attended^T over INNER (S0 steps of 16).
     {
-      constexpr int PD = NI > 3 ? 2 : 4;  // weight fragments prefetched this many steps ahead
+      constexpr int PD = kPdOut;  // weight fragments prefetched this many steps ahead
       u32x4 a[PD][NI];
       auto load_a = [&](int s, u32x4 (&dst)[NI]) {
 #pragma unroll
@@ -260,7 +262,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void block_tail_kernel(TailParams p
           }
         }
       {
-        constexpr int PD = NB > 1 ? 4 : 8;
+        constexpr int PD = kPdIn;
         const int blk0 = (kCH / 32) * c + NB * fq;
         u32x4 a[PD][NB];
         auto load_a = [&](int s, u32x4 (&dst)[NB]) {
@@ -311,7 +313,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void block_tail_kernel(TailParams p
       __syncthreads();
       // FF out: acc += W2^T . h^T over the chunk's kCH hidden units (kSC steps of 16).
       {
-        constexpr int PD = NI > 3 ? 2 : 4;
+        constexpr int PD = kPdOut;
         const int sh = hidden / 16;
         u32x4 a[PD][NI];
         auto load_a = [&](int s, u32x4 (&dst)[NI]) {
