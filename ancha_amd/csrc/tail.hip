@@ -30,7 +30,7 @@
 // registers, and on gfx950 the store's first dword then came out as the new value in some lanes, now
 // and then.
 //
-// Workgroup: 32 NJ rows (64; 32 in calls with few rows), 4 waves, one per feature quarter (and
+// Workgroup: 32 NJ rows (64; 32 or 96 in smaller calls), 4 waves, one per feature quarter (and
 // SIMD); two workgroups per CU, whose phases drift apart, so one's GELU / norm VALU work runs beside
 // the other's MFMAs. The out accumulator (rows x dim) stays in registers from the residual load to the final store; the
 // hidden dimension runs in chunks of 256 units up to dim 384, 128 at dim 512 (per chunk: FF-in
@@ -78,7 +78,7 @@ __device__ __forceinline__ void row_totals(float* red, const float (&part)[NJ], 
 
 // DIM = 128 * NI features, INNER = heads * 64.
 template <int NI, int INNER, int NJ>
-__global__ __launch_bounds__(kWaves * 64, 2) void block_tail_kernel(TailParams p) {
+__global__ __launch_bounds__(kWaves * 64, NJ > 2 ? 1 : 2) void block_tail_kernel(TailParams p) {
   constexpr int kRows = 32 * NJ;  // rows per workgroup step
   // k steps of weight fragments in flight, out projection / FF out and FF in (twice to three times
   // as many with one row block: parity at dim 384, 69 against 66 us at dim 512).
@@ -473,6 +473,15 @@ hipError_t launch_t(const TailParams& p, hipStream_t stream) {
     return hipGetLastError();
   }
   const int blocks = (p.rows + 63) / 64;  // two workgroups per CU
+  // Just past one 64-row workgroup per CU the few CUs with two set the time; 96-row workgroups (one
+  // a CU, one wave per SIMD) then still fit one per CU: 18 060 rows 91.4 -> 81.9 us (dim 512 144.5 ->
+  // 125.1), 24 576 rows 97.7 -> 95.6 (159 -> 148). At 16 384 rows they would be 78.9 against 66.2, at
+  // 28 000 153 against 105; 128-row workgroups up to 32 768 rows 97.6 at 18 060, 120 against 118.
+  if (blocks > cus && (p.rows + 95) / 96 <= cus) {
+    hipLaunchKernelGGL((block_tail_kernel<NI, INNER, 3>), dim3((p.rows + 95) / 96),
+                       dim3(kWaves * 64), 0, stream, p);
+    return hipGetLastError();
+  }
   hipLaunchKernelGGL((block_tail_kernel<NI, INNER, 2>), dim3(blocks < 2 * cus ? blocks : 2 * cus),
                      dim3(kWaves * 64), 0, stream, p);
   return hipGetLastError();

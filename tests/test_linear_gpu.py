@@ -212,10 +212,11 @@ def test_block_attention_core_at_layer_pair_shape(gpu, axis):
     assert err < 2e-3
 
 
-@pytest.mark.parametrize("dim,groups", [(384, (1, 150, 300, 1200)), (512, (1, 60, 150, 900))])
+@pytest.mark.parametrize("dim,groups", [(384, (1, 150, 300, 600, 1200)), (512, (1, 60, 150, 700, 900))])
 def test_block_rows_do_not_depend_on_the_call_size(gpu, dim, groups):
     """A sequence's rows are computed alike however many row blocks a call has: the projection's
-    columns split over six, three, two and one workgroups give the same bits."""
+    columns split over six, three, two and one workgroups and the tail's 32-, 64- and 96-row
+    workgroups give the same bits."""
     w = _block_weights(dim, 8, 4 * dim)
     block = roformer.Transformer(w, gpu)
     tokens = 33
