@@ -425,7 +425,8 @@ bool attention_grid_fits(size_t groups, size_t tokens, size_t heads) {
   const size_t problems = groups * heads;
   if (groups != 0 && problems / groups != heads) return false;
   // T <= 64: one 256-thread workgroup per problem at most. T > 64: the long-sequence kernel's
-  // 512-query passes are counted in an int (its grid is at most twice the CU count).
+  // 512-query passes are counted in an int (its grid is at most twice the CU count, or below 2^23
+  // workgroups of 256 threads where it takes 128-query passes).
   const size_t blocks = tokens <= 64 ? problems : problems * ((tokens + 511) / 512);
   const size_t threads = tokens <= 64 ? 256 : 1024;
   return blocks < (size_t(1) << 31) && (tokens > 64 || blocks * threads < (size_t(1) << 32));

@@ -14,6 +14,9 @@
 // step the next tile's K / V rows are requested first and its table rows (and the query chunk)
 // after the first 32-key block, so the 16 waves' requests do not all queue at once.
 //
+// Short sequences and calls of few problems take the same kernel with 4 waves: 128 queries a
+// workgroup, two or three workgroups a CU, one pass each (launch_t says where and what it measured).
+//
 // The softmax VALU work (exp2, max, fp16 packing) costs about as many cycles as the MFMAs, so
 // the kernel is built for overlap: at most 128 VGPRs, which puts four waves on every SIMD, one
 // wave's softmax running beside another's MFMAs.
