@@ -170,7 +170,12 @@ def _linear(x: torch.Tensor, weight: torch.Tensor, epilogue: Epilogue,
     out = x.new_empty((n, m))
     lib = _native.lib()
     need = lib.ancha_amd_linear_workspace(n, k, m)
-    workspace = torch.empty(need, device=x.device, dtype=torch.uint8) if need else None
+    workspace = None
+    if need:
+        try:
+            workspace = x.new_empty(need, dtype=torch.uint8)
+        except torch.OutOfMemoryError:
+            need = 0  # the kernel without scratch
     rc = lib.ancha_amd_linear(
         x.data_ptr(), n, k, x.stride(0), w.data_ptr(), m, _ptr(bias), int(epilogue.gelu),
         _ptr(table), tokens, width, _ptr(residual), int(norm), _ptr(workspace), need,
