@@ -38,12 +38,14 @@ namespace {
 constexpr int kWaves = 8;
 constexpr int kFrag = 1024;
 
-// After a 16-byte store with its scalar offset in a register: a wait state before anything can reuse
-// the data registers. The compiler leaves none there, and on gfx950 the store's first dword then came
-// out as the new value in some lanes (dropping the scalar offset instead spills here).
+// After a 16-byte store with its scalar offset in a register: two wait states, what gfx950 needs
+// before a vector instruction rewrites the data registers of a store of more than 8 bytes. The
+// compiler keeps them where the scalar offset is a constant and leaves none here; the store's first
+// dword then came out as the new value in some lanes (dropping the scalar offset instead spills).
+// tests/test_wide_stores.py counts them in the built library.
 __device__ __forceinline__ void store_gap() {
   __builtin_amdgcn_sched_barrier(0);
-  asm volatile("s_nop 0");
+  asm volatile("s_nop 1");
   __builtin_amdgcn_sched_barrier(0);
 }
 

@@ -25,10 +25,10 @@
 // row pieces. A lane per row (16-byte pieces of 32 rows an access, as the accumulators and the
 // fragments have them) costs the address unit four times the cycles, and the weight loads of the
 // other workgroup wait behind it: 362 -> 336 us per call at 96 120 rows, dim 384 (341 -> 324 without
-// the fp16 output), 98 -> 90 us at 18 060 rows. The 16-byte stores have no scalar offset: with one,
-// the compiler leaves no wait state between the store and an instruction that reuses its data
-// registers, and on gfx950 the store's first dword then came out as the new value in some lanes, now
-// and then.
+// the fp16 output), 98 -> 90 us at 18 060 rows. The 16-byte stores have no scalar offset: with one
+// in a register, the compiler leaves out the two wait states that gfx950 needs between the store and
+// an instruction that rewrites its data registers, and the store's first dword then came out as the
+// new value in some lanes, now and then.
 //
 // Workgroup: 32 NJ rows (64; 32 or 96 in smaller calls), 4 waves, one per feature quarter (and
 // SIMD); two workgroups per CU, whose phases drift apart, so one's GELU / norm VALU work runs beside
