@@ -64,10 +64,12 @@ SIGNATURES = {
     "ancha_hip_istft_noalloc": (_int, [_p, _p, _sz, _sz, _sz, _int, _p, _p]),
     "ancha_hip_check": (_int, []),
     "ancha_hip_last_error": (ctypes.c_char_p, []),
-    # Not in the header: linear / norm_linear with scratch for the weight's fp16 fragments.
+    # Not in the header: linear / norm_linear with scratch for the weight's fp16 fragments, and the
+    # attention kernels' split, for the tests.
     "ancha_amd_linear_workspace": (_sz, [_sz, _sz, _sz]),
     "ancha_amd_linear": (_int, [_p, _sz, _sz, _sz, _p, _sz, _p, _int, _p, _sz, _sz, _p, _int, _p,
                                 _sz, _p, _p]),
+    "ancha_amd_attention_queries": (_int, [_sz, _sz, _sz, _int, _int]),
 }
 
 

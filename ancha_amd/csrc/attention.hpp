@@ -47,7 +47,7 @@ __device__ __forceinline__ OutRows out_rows(const AttnParams& p, int g, int h) {
   return o;
 }
 
-// Long sequences (T > 64) on v_mfma_f32_32x32x16_f16: 16 waves x 32 queries per workgroup.
+// Long sequences (T > 64) on v_mfma_f32_32x32x16_f16: 16 or 4 waves x 32 queries per workgroup.
 // fp32 q / k / v (`aligned`: rows, table and output 16-byte aligned; otherwise 4-byte accesses),
 // or the block's fp16 projection (in_half, aligned only).
 hipError_t launch_attention_long(const AttnParams& p, bool gated, bool rope, bool aligned,

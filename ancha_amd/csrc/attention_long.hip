@@ -15,7 +15,8 @@
 // after the first 32-key block, so the 16 waves' requests do not all queue at once.
 //
 // Short sequences and calls of few problems take the same kernel with 4 waves: 128 queries a
-// workgroup, two or three workgroups a CU, one pass each (launch_t says where and what it measured).
+// workgroup, two or three workgroups a CU, one pass each (attention_short_passes says where and
+// what it measured).
 //
 // The softmax VALU work (exp2, max, fp16 packing) costs about as many cycles as the MFMAs, so
 // the kernel is built for overlap: at most 128 VGPRs, which puts four waves on every SIMD, one
@@ -624,32 +625,49 @@ __global__ __launch_bounds__(NW * 64, NW == 16 ? 1 : XH || (!ROPE && ALIGNED) ? 
   }
 }
 
+}  // namespace
+
+// Where 128-query passes on 4-wave workgroups (none walking) are ahead of 512-query ones. Times are
+// groups x tokens x 8 heads, 512-query -> 128-query passes, every line read off sweeps of 129 - 1722
+// tokens and 8 - 2400 problems with each form forced:
+// - Up to 128 queries, where a 512-query workgroup has four waves busy of sixteen: 200 x 100 52.5 ->
+//   31.8 us, with rotary 58.2 -> 39.0, 600 x 65 168 -> 70.
+// - Aligned rows with nothing to rotate on load, three 4-wave workgroups a CU: within one round of
+//   512-query passes up to two of them a CU (1 x 801 33.9 -> 19.5, 16 x 512 27.8 -> 22.5; beyond, 25 x
+//   450 28.9 -> 34.5, 15 x 801 39.2 -> 48.6); past that round up to 384 tokens (200 x 256 119.7 -> 91)
+//   or five a CU (20 x 801 70.4 -> 56.9, 10 x 1722 126.8 -> 106.9; 60 x 801 would be 147 -> 161:
+//   more K / V traffic per query).
+// - Otherwise two or fewer a CU (rotary rows: every K row is rotated once per 128 queries; unaligned
+//   rows: 4-byte accesses), so up to one a CU (unaligned 3 x 1025 47.6 -> 41.0, but 4 x 1025, 288 of
+//   them, 47.7 -> 63.0; aligned rows past 256 tokens an eighth more, 3 x 1301 55 -> 42). At 129 - 256
+//   tokens also where the last round of 512-query passes is at most half full (rotary 80 x 200 41.8 ->
+//   36.4, 200 x 200 108.7 -> 102.2, unaligned 80 x 256 54.7 -> 49.0; else rotary 50 x 129 23.3 ->
+//   25.2, unaligned 50 x 256 33.0 -> 35.0), except unaligned rows with a rotary table (200 x 256 146
+//   -> 153).
+bool attention_short_passes(long problems, long tokens, bool rotated, bool aligned) {
+  const long cus = device_cus();
+  const long passes = problems * ((tokens + 511) / 512), tiles = problems * ((tokens + 127) / 128);
+  if (tiles >= 1l << 23) return false;  // 256 threads each: below HIP's 2^32 threads
+  if (tokens <= 128) return true;
+  if (aligned && !rotated) return passes <= cus ? tiles <= 2 * cus : tokens <= 384 || tiles <= 5 * cus;
+  if (tiles <= (aligned && tokens > 256 ? cus + cus / 8 : cus)) return true;
+  return (aligned || !rotated) && tokens <= 256 && passes > cus && (passes - 1) % cus < cus / 2;
+}
+
+namespace {
+
 template <bool GATED, bool ROPE, bool XH, bool ALIGNED = true, bool TALIGNED = ALIGNED>
 hipError_t launch_t(const AttnParams& p, hipStream_t stream) {
   const int problems = p.groups * p.heads;
+  if (attention_short_passes(problems, p.tokens, ROPE && !XH, ALIGNED)) {
+    const int qb = (p.tokens + 127) / 128, tiles = problems * qb;
+    hipLaunchKernelGGL((attention_long_kernel<GATED, ROPE, XH, ALIGNED, TALIGNED, 4>), dim3(tiles),
+                       dim3(256), 0, stream, p, qb, tiles);
+    return hipGetLastError();
+  }
   const int qblocks = (p.tokens + 511) / 512;
   const int passes = problems * qblocks;
   const int cus = device_cus();
-  // 128-query passes on 4-wave workgroups (three a CU, two with fp32 rotary rows), none walking:
-  // up to 128 queries, where a 512-query workgroup has four waves busy of sixteen (200 x 100 x 8
-  // heads: 52.5 -> 31.8 us, with rotary 58.2 -> 39.0, 600 x 65 x 8 168 -> 70); with up to about one
-  // workgroup per CU (1 x 801 x 8 33.2 -> 19.3, 4 x 256 x 8 12.6 -> 10.0); and without rotary rows
-  // up to 384 tokens (200 x 256 x 8 120 -> 93, 60 x 301 x 8 40.2 -> 36.6) or five workgroups per CU
-  // (20 x 801 x 8 73 -> 60; 60 x 801 x 8 would be 161 against 147: more K / V traffic per query).
-  // With rotary rows every K row is rotated once per 128 queries: 129 - 256 tokens gain only from
-  // three workgroups per CU on (200 x 200 x 8 112 -> 105; 20 x 200 x 8 16.4 against 15.2), longer
-  // ones lose (60 x 400 x 8 79 against 62).
-  const int qb = (p.tokens + 127) / 128;
-  const long tiles = (long)problems * qb;
-  const bool heavy = ROPE && !XH;
-  const bool few = p.tokens <= 128 || tiles <= cus + cus / 8 ||
-                   (heavy ? p.tokens <= 256 && tiles >= 3l * cus
-                          : p.tokens <= 384 || tiles <= 5l * cus);
-  if (few && tiles < (1l << 23)) {  // 256 threads each: below HIP's 2^32 threads
-    hipLaunchKernelGGL((attention_long_kernel<GATED, ROPE, XH, ALIGNED, TALIGNED, 4>),
-                       dim3((unsigned)tiles), dim3(256), 0, stream, p, qb, (int)tiles);
-    return hipGetLastError();
-  }
   // One workgroup per CU walks the passes when there are more than two rounds of them; fewer
   // passes run one per workgroup (the walk would only lengthen the critical path).
   const int grid = passes <= 2 * cus ? passes : cus;

@@ -317,6 +317,14 @@ int ancha_hip_gated_attention(const float* packed, size_t groups, size_t tokens,
   return run_attention(p, groups, tokens, heads, stream, "ancha_hip_gated_attention");
 }
 
+// For the tests: queries per workgroup of an attention call with T > 64 tokens (128 or 512).
+int ancha_amd_attention_queries(size_t groups, size_t tokens, size_t heads, int rotated, int aligned) {
+  return ancha::attention_short_passes(static_cast<long>(groups * heads), static_cast<long>(tokens),
+                                       rotated != 0, aligned != 0)
+             ? 128
+             : 512;
+}
+
 int ancha_hip_check(void) { return g_sticky.load(); }
 
 const char* ancha_hip_last_error(void) { return g_last.c_str(); }

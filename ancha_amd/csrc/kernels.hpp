@@ -42,6 +42,9 @@ hipError_t launch_attention(const AttnParams& p, bool aligned, hipStream_t strea
 // Whether the launch launch_attention picks for this shape fits HIP's grid limits (workgroup
 // count below 2^31 and total thread count below 2^32).
 bool attention_grid_fits(size_t groups, size_t tokens, size_t heads);
+// Whether a call of T > 64 tokens runs in 128-query passes (4 waves) instead of 512-query ones (16):
+// `rotated` fp32 rows with a rotary table, `aligned` as launch_attention's.
+bool attention_short_passes(long problems, long tokens, bool rotated, bool aligned);
 
 // out = epilogue(x . w): x [n, k] (row stride ldx), w [k, m] row-major (the reference's
 // [in, out] Linear layout), out [n, m] contiguous. Epilogue, in order: optional input row norm

@@ -15,7 +15,7 @@ import pytest
 import torch
 
 import oracle as O
-from ancha_amd import fused
+from ancha_amd import _native, fused
 from ancha_amd import workload as W
 
 pytestmark = pytest.mark.gpu
@@ -297,27 +297,34 @@ def test_tail_keys_are_attended_and_padding_is_masked(gpu, tokens):
     check(f"tail keys T={tokens}", got, expected)
 
 
-@pytest.mark.parametrize("groups,tokens,rope", [(41, 400, False), (33, 513, False), (22, 801, False),
-                                                (40, 130, True), (36, 256, True), (10, 801, True)])
-def test_small_and_walking_workgroups_agree(gpu, groups, tokens, rope):
+# Rounds of 512-query passes of the whole call: one pass per workgroup up to two rounds, a walk beyond.
+@pytest.mark.parametrize("tokens,rope,aligned,rounds", [
+    (400, False, True, 0.75), (400, False, True, 2.1), (513, False, True, 2.1),
+    (801, False, True, 1.75), (801, False, True, 2.1), (130, True, True, 1.75),
+    (130, True, True, 2.75), (801, True, True, 0.4), (801, True, True, 2.1),
+    (200, False, False, 0.75), (301, False, False, 2.1), (200, True, False, 1.75),
+    (401, True, False, 2.1)])
+def test_small_and_walking_workgroups_agree(gpu, tokens, rope, aligned, rounds):
     """A call large enough for the 16-wave workgroups and its first groups alone, which take the
     4-wave ones: both run the same arithmetic per 32 queries, so the same bits; oracle on a sample."""
-    q, k, v = (dev(W.normal((groups, tokens, 8, 64), s, 1.0), gpu) for s in (61, 62, 63))
+    heads, few = 8, 2
+    cus = torch.cuda.get_device_properties(gpu).multi_processor_count
+    groups = math.ceil(rounds * cus / (heads * math.ceil(tokens / 512)))
+    queries = lambda g: _native.lib().ancha_amd_attention_queries(g, tokens, heads, rope, aligned)
+    assert (queries(groups), queries(few)) == (512, 128)
+    columns = heads * 64 if aligned else heads * 64 + 1
+    gen = torch.Generator(device=gpu).manual_seed(61)
+    q, k, v = (torch.randn(groups, tokens, columns, generator=gen, device=gpu)[..., :heads * 64]
+               .unflatten(2, (heads, 64)) for _ in range(3))
     table = W.axis_rope_packed(W.rope_freqs(), tokens) if rope else None
     if not rope:
-        q = q / 8
+        q *= 0.125
     t = dev(table, gpu) if rope else None
     whole = fused.attention(q, k, v, rope=t)
-    few = 2 if tokens > 256 else 4
-    part = fused.attention(q[:few].contiguous(), k[:few].contiguous(), v[:few].contiguous(), rope=t)
+    part = fused.attention(q[:few], k[:few], v[:few], rope=t)
     assert torch.equal(part, whole[:few])
-    qn, kn, vn = (a[:1, :, :1].cpu().numpy() for a in (q, k, v))
-    if rope:
-        want = O.attention_op(np.ascontiguousarray(qn), np.ascontiguousarray(kn),
-                              np.ascontiguousarray(vn), rope=table)
-    else:
-        want = O.attention_op(np.ascontiguousarray(qn), np.ascontiguousarray(kn),
-                              np.ascontiguousarray(vn))
+    qn, kn, vn = (np.ascontiguousarray(a[:1, :, :1].cpu().numpy()) for a in (q, k, v))
+    want = O.attention_op(qn, kn, vn, rope=table) if rope else O.attention_op(qn, kn, vn)
     check(f"T={tokens}", whole[:1, :, :1].cpu().numpy(), want)
 
 
