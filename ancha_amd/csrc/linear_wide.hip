@@ -400,46 +400,72 @@ void launch_stream(const LinearParams& p, hipStream_t stream) {
     hipLaunchKernelGGL((linear_stream_kernel<NI, RB, 2>), grid, block, 0, stream, p, groups);
 }
 
-}  // namespace
+// The form a call takes (kGeneral: linear.hip).
+enum class Form { kGeneral, kTile32x128, kTile64x128, kTile128x128, kTile96x384, kTile64x512, kResident };
 
-size_t linear_wide_workspace(size_t n, size_t k, size_t m) {
-  if (n == 0 || k == 0 || m == 0 || k % 128 || m % 128) return 0;
-  return k * m * 2;
-}
-
-hipError_t launch_linear_wide(const LinearParams& params, void* workspace, hipStream_t stream) {
-  LinearParams p = params;
-  const int frags = (p.m / 32) * (p.k / 16);
-  hipLaunchKernelGGL(weight_fragments_kernel, dim3((frags + 3) / 4), dim3(256), 0, stream, p.w, p.k,
-                     p.m, static_cast<u32x4*>(workspace));
-  p.w = static_cast<const float*>(workspace);  // fp16 fragments from here on
+Form choose(long n, long k, long m) {
+  if (k % 128 || m % 128) return Form::kGeneral;
+  const long cus = device_cus();
+  const long small = (n + 63) / 64 * (m / 128);     // 64 x 128 tiles
+  const long general = (n + 127) / 128 * (m / 128);  // 128 x 128 ones, linear.hip's too
+  // Few rows on a very wide weight: laying it out costs more than it saves where linear.hip already
+  // fills the chip (200 x 256 -> 16384 17.7 against 20.6 us, 500 x 512 -> 16384 29.7 against 34.5).
+  if (m >= 8192 && k <= 512 && n <= 512 && 2 * general > cus) return Form::kGeneral;
   // Few tiles: the smallest ones, to use the chip at all (up to two 64 x 128 tiles per CU the stream
   // form is ahead also where the resident one applies: 300 x 384 -> 1664 6.0 against 12.5 us,
   // 1000 x 384 -> 1664 8.6 against 12.9). Then the resident form for wide outputs (x is read once), else the
   // widest stream tile that gives at least half the CUs a workgroup: 18 060 x 1536 -> 384 runs at 47
   // us in 96 x 384 tiles, 64 in 64 x 384 (a second round), 62 in 128 x 128.
-  const int cus = device_cus();
-  const long small = (long)((p.n + 63) / 64) * (p.m / 128);  // 64 x 128 tiles
-  // Row blocks of 96 times column groups, and 64 x 512 tiles.
-  const long wide3 = (long)((p.n + 95) / 96) * (p.m / 384);
-  const long wide4 = (long)((p.n + 63) / 64) * (p.m / 512);
-  if (2 * small <= cus) {
-    launch_stream<1, 1>(p, stream);
-  } else if (small <= 2 * cus) {
-    launch_stream<1, 2>(p, stream);
-  } else if (p.m > 512 && (p.k == 128 || p.k == 256 || p.k == 384 || p.k == 512)) {
-    switch (p.k) {
-      case 128: launch_resident<8>(p, stream); break;
-      case 256: launch_resident<16>(p, stream); break;
-      case 384: launch_resident<24>(p, stream); break;
-      default: launch_resident<32>(p, stream);
-    }
-  } else if (p.m % 384 == 0 && 2 * wide3 >= cus) {
-    launch_stream<3, 3>(p, stream);
-  } else if (p.m % 512 == 0 && 2 * wide4 >= cus) {
-    launch_stream<4, 2>(p, stream);
-  } else {
-    launch_stream<1, 4>(p, stream);
+  if (2 * small <= cus) return Form::kTile32x128;
+  if (small <= 2 * cus) return Form::kTile64x128;
+  if (m > 512 && (k == 128 || k == 256 || k == 384 || k == 512)) return Form::kResident;
+  if (m % 384 == 0 && 2 * ((n + 95) / 96 * (m / 384)) >= cus) return Form::kTile96x384;
+  if (m % 512 == 0 && 2 * ((n + 63) / 64 * (m / 512)) >= cus) return Form::kTile64x512;
+  // What is left has 128 x 128 tiles either way, here one workgroup per CU against linear.hip's two. Here is
+  // ahead with a long k and either enough tiles that the rounds' ends do not count (33 000 x 640 -> 1664
+  // 225 -> 189 us), just more than one round of linear.hip's (40 000 x 1024 -> 256 83 -> 72), or an x of
+  // 112 MiB and more, which linear.hip reads again for every column group (40 000 x 1536 -> 128
+  // 82 -> 67). Elsewhere linear.hip: 65 000 x 256 -> 256 34 against 48, 24 576 x 1024 -> 256 37 against
+  // 46, 10 500 x 640 -> 640 27 against 33, 20 000 x 640 -> 1664 103 against 121.
+  const bool large = n * k * 4 >= (112l << 20) && (k >= 1536 || general > 2 * cus);
+  if (k > 512 && (general >= 8 * cus || (general > 2 * cus && general <= 3 * cus) || large))
+    return Form::kTile128x128;
+  return Form::kGeneral;
+}
+
+}  // namespace
+
+size_t linear_wide_workspace(size_t n, size_t k, size_t m) {
+  // Past these sizes the call is refused.
+  if (n == 0 || k == 0 || m == 0 || n > 0x7fffffff || m >= (size_t(1) << 22) ||
+      k >= (size_t(1) << 30) / m)
+    return 0;
+  return choose((long)n, (long)k, (long)m) == Form::kGeneral ? 0 : k * m * 2;
+}
+
+hipError_t launch_linear_wide(const LinearParams& params, void* workspace, hipStream_t stream) {
+  LinearParams p = params;
+  const Form form = choose(p.n, p.k, p.m);
+  if (form == Form::kGeneral) return hipErrorInvalidValue;  // linear_wide_workspace gave 0
+  const int frags = (p.m / 32) * (p.k / 16);
+  hipLaunchKernelGGL(weight_fragments_kernel, dim3((frags + 3) / 4), dim3(256), 0, stream, p.w, p.k,
+                     p.m, static_cast<u32x4*>(workspace));
+  p.w = static_cast<const float*>(workspace);  // fp16 fragments from here on
+  switch (form) {
+    case Form::kTile32x128: launch_stream<1, 1>(p, stream); break;
+    case Form::kTile64x128: launch_stream<1, 2>(p, stream); break;
+    case Form::kTile128x128: launch_stream<1, 4>(p, stream); break;
+    case Form::kTile96x384: launch_stream<3, 3>(p, stream); break;
+    case Form::kTile64x512: launch_stream<4, 2>(p, stream); break;
+    case Form::kResident:
+      switch (p.k) {
+        case 128: launch_resident<8>(p, stream); break;
+        case 256: launch_resident<16>(p, stream); break;
+        case 384: launch_resident<24>(p, stream); break;
+        default: launch_resident<32>(p, stream);
+      }
+      break;
+    case Form::kGeneral: break;
   }
   return hipGetLastError();
 }

@@ -30,3 +30,23 @@ ATTENTION = [
 @pytest.mark.parametrize("groups,tokens,rotated,aligned,queries", ATTENTION)
 def test_attention_passes(groups, tokens, rotated, aligned, queries):
     assert _native.lib().ancha_amd_attention_queries(groups, tokens, 8, rotated, aligned) == queries
+
+
+# n, k, m, whether the weight is laid out first (scratch of k m halves)
+LINEAR = [
+    (32, 384, 1664, True), (300, 1536, 384, True), (96120, 384, 1664, True), (18060, 1536, 384, True),
+    (9000, 384, 512, True), (33000, 640, 1664, True), (40000, 1024, 256, True), (40000, 1536, 128, True),
+    # 128 x 128 tiles that linear.hip runs two to a CU.
+    (65000, 256, 256, False), (32000, 512, 256, False), (24576, 1024, 256, False),
+    (10500, 640, 640, False), (20000, 640, 1664, False), (96120, 128, 128, False),
+    # Few rows on a very wide weight.
+    (200, 256, 16384, False), (500, 512, 16384, False), (128, 256, 8192, True), (700, 512, 16384, True),
+    # Shapes that only linear.hip takes, and calls that are refused.
+    (1000, 384, 200, False), (1000, 64, 128, False), (0, 384, 384, False), (1 << 31, 384, 384, False),
+    (4, 128, 1 << 22, False), (4, 1 << 23, 128, False),
+]
+
+
+@pytest.mark.parametrize("n,k,m,laid_out", LINEAR)
+def test_linear_scratch(n, k, m, laid_out):
+    assert _native.lib().ancha_amd_linear_workspace(n, k, m) == (2 * k * m if laid_out else 0)

@@ -359,13 +359,15 @@ def test_block_odd_head_count(gpu, tokens, heads):
     assert err < 2e-3
 
 
-# One case per tile form of the prepared-weight path and its edges: row blocks of 32 / 64 / 96 / 128
-# with a ragged last one, two and four k tiles in flight, one and several column groups, and the
-# resident form with its columns split and whole.
+# One case per form of the prepared-weight path (256 CUs) and its edges: row blocks of 32 / 64 / 96 / 128
+# with a ragged last one, two and four k tiles in flight, one and several column groups; the resident
+# form with its columns split (k of 128 - 512) and with more row blocks than CUs, so that a workgroup
+# takes a second one.
 @pytest.mark.parametrize("n,k,m,ldx", [
     (1, 128, 128, 128), (33, 384, 1664, 388), (65, 640, 512, 640), (300, 1536, 384, 1536),
     (2001, 512, 384, 516), (2600, 128, 1536, 128), (5000, 256, 1152, 256), (4003, 384, 1664, 384),
-    (2700, 512, 2048, 512), (12301, 256, 384, 256), (8200, 384, 512, 384), (16500, 128, 256, 128)])
+    (2700, 512, 2048, 512), (12301, 256, 384, 256), (8200, 384, 512, 384), (16500, 128, 256, 128),
+    (5130, 640, 1664, 644), (7001, 128, 640, 132), (25001, 128, 640, 128)])
 def test_prepared_weight_tiles(gpu, n, k, m, ldx):
     rng = np.random.default_rng(5)
     base = rng.standard_normal((n, ldx)).astype(np.float32)
@@ -385,9 +387,11 @@ def test_prepared_weight_tiles(gpu, n, k, m, ldx):
     got = fused.norm_linear(X, Wt, fused.Epilogue(bias=B, gelu=True)).cpu().numpy()
     check("norm + bias + GELU", got[rows], O.linear(xn, w, bias=b, gelu=True),
           bound(xn, w, 1.13) + 1e-6)
-    # Rotary columns end inside the matrix; n tokens, so a row's token is the row.
+    # Rotary columns end inside the matrix; the tokens repeat (n has a divisor) or are the rows.
     width = m // 128 * 64 if m > 128 else 64
-    table = W.axis_rope_packed(W.rope_freqs(), n)
-    got = fused.linear(X, Wt, fused.Epilogue(rotary=(dev(table, gpu), width))).cpu().numpy()
-    want = O.linear(xs, w, rope=np.ascontiguousarray(table[:, rows]), tokens=len(rows), width=width)
-    check("rotary", got[rows], want, bound(xs, w, 1.42) + 1e-6)
+    tokens = next((n // d for d in range(2, 64) if n % d == 0), n)
+    table = W.axis_rope_packed(W.rope_freqs(), tokens)
+    got = fused.norm_linear(X, Wt, fused.Epilogue(rotary=(dev(table, gpu), width))).cpu().numpy()
+    want = O.linear(xn, w, rope=np.ascontiguousarray(table[:, rows % tokens]), tokens=len(rows),
+                    width=width)
+    check("norm + rotary", got[rows], want, bound(xn, w, 1.42) + 1e-6)
