@@ -16,7 +16,7 @@ import pytest
 import torch
 
 import oracle as O
-from ancha_amd import fused, roformer
+from ancha_amd import _native, fused, roformer
 from ancha_amd import workload as W
 from tests.golden import cases as C
 
@@ -128,7 +128,8 @@ def test_unit_norm(gpu, rows, dim, scaled):
 # odd strides, a row count that ends inside a wave's rows, and the first length past the registers.
 @pytest.mark.parametrize("rows,dim,pad", [
     (7, 4, 0), (5, 128, 0), (9, 132, 4), (33, 384, 0), (3, 388, 0), (6, 516, 12), (2, 1024, 0),
-    (3, 1028, 0), (1, 1, 0), (5, 65, 3), (9, 129, 0), (3, 400, 1), (7, 511, 0), (3, 640, 1),
+    (3, 1028, 0), (1, 1, 0), (5, 65, 3), (9, 129, 0), (5, 259, 0), (3, 383, 1), (3, 384, 1),
+    (3, 400, 1), (7, 511, 0), (3, 640, 1),
     (2, 767, 0), (5, 1023, 2), (3, 1025, 0)])
 def test_unit_norm_row_lengths(gpu, rows, dim, pad):
     base = W.normal((rows, dim + pad), 43, 3.0)
@@ -212,14 +213,20 @@ def test_block_attention_core_at_layer_pair_shape(gpu, axis):
     assert err < 2e-3
 
 
-@pytest.mark.parametrize("dim,groups", [(384, (1, 150, 300, 600, 1200)), (512, (1, 60, 150, 700, 900))])
-def test_block_rows_do_not_depend_on_the_call_size(gpu, dim, groups):
-    """A sequence's rows are computed alike however many row blocks a call has: the projection's
-    columns split over six, three, two and one workgroups and the tail's 32-, 64- and 96-row
-    workgroups give the same bits."""
-    w = _block_weights(dim, 8, 4 * dim)
+# Rows of the call per CU. Projection, in row blocks of 128 (96 at dim 512): columns split over six, three
+# and two workgroups, one workgroup with a row tile less, whole blocks in more than one round (dim 128
+# has too few columns to split). Tail: 32 rows a workgroup up to 32 per CU, 64, 96 just past 64, 64.
+@pytest.mark.parametrize("dim,heads,rows", [(384, 8, (18, 36, 52, 78, 155)),
+                                            (512, 8, (14, 27, 39, 52, 78, 110)),
+                                            (256, 8, (78, 155)), (128, 2, (78, 155))])
+def test_block_rows_do_not_depend_on_the_call_size(gpu, dim, heads, rows):
+    """A sequence's rows are computed alike however many row blocks a call has: every split of the
+    projection and every workgroup size of the tail give the same bits."""
+    w = _block_weights(dim, heads, 4 * dim)
     block = roformer.Transformer(w, gpu)
     tokens = 33
+    cus = torch.cuda.get_device_properties(gpu).multi_processor_count
+    groups = [1] + [-(-r * cus // tokens) for r in rows]
     table = roformer.axis_rope(w["freqs"], tokens, gpu)
     x = dev(W.normal((groups[-1], tokens, dim), 71, 1.0), gpu)
     whole = block(x, table)
@@ -395,3 +402,50 @@ def test_prepared_weight_tiles(gpu, n, k, m, ldx):
     want = O.linear(xn, w, rope=np.ascontiguousarray(table[:, rows % tokens]), tokens=len(rows),
                     width=width)
     check("norm + rotary", got[rows], want, bound(xn, w, 1.42) + 1e-6)
+
+
+@pytest.mark.parametrize("n,k,m", [(33, 384, 1664), (300, 1536, 384), (4003, 256, 1152)])
+def test_linear_without_scratch(gpu, monkeypatch, n, k, m):
+    """Without (enough) scratch for the laid-out weight a call runs linear.hip: the C entry with a null
+    and with a short workspace, and the Python op when the allocation of the scratch fails, give its
+    bits, within the bound of the oracle."""
+    lib = _native.lib()
+    need = lib.ancha_amd_linear_workspace(n, k, m)
+    assert need == 2 * k * m
+    x, w = W.normal((n, k), 51, 1.0), W.normal((k, m), 52, 0.05)
+    b, r = W.normal((m,), 53, 0.1), W.normal((n, m), 54, 1.0)
+    table = W.axis_rope_packed(W.rope_freqs(), n)
+    X, Wt, B, R, Tb = (dev(a, gpu) for a in (x, w, b, r, table))
+    scratch = torch.empty(need, dtype=torch.uint8, device=gpu)
+    xn, width = O.unit_norm(x), m // 128 * 64
+    stream = torch.cuda.current_stream().cuda_stream
+    new_empty = torch.Tensor.new_empty
+
+    def no_scratch(self, *args, **kwargs):
+        if kwargs.get("dtype") == torch.uint8:
+            raise torch.OutOfMemoryError("no scratch")
+        return new_empty(self, *args, **kwargs)
+
+    for norm, gelu, rope, residual in ((0, 0, None, R), (1, 1, None, None), (0, 0, Tb, None)):
+        ptr = lambda t: None if t is None else t.data_ptr()
+        tokens = 0 if rope is None else n
+        outs = [torch.full((n, m), float("nan"), device=gpu) for _ in range(3)]
+        entry = lib.ancha_hip_norm_linear if norm else lib.ancha_hip_linear
+        common = (X.data_ptr(), n, k, k, Wt.data_ptr(), m, B.data_ptr(), gelu, ptr(rope), tokens,
+                  width if tokens else 0, ptr(residual))
+        assert entry(*common, outs[0].data_ptr(), stream) == 0
+        assert lib.ancha_amd_linear(*common, norm, None, 0, outs[1].data_ptr(), stream) == 0
+        assert lib.ancha_amd_linear(*common, norm, scratch.data_ptr(), need - 1, outs[2].data_ptr(),
+                                    stream) == 0
+        op = fused.norm_linear if norm else fused.linear
+        epilogue = fused.Epilogue(bias=B, gelu=bool(gelu), residual=residual,
+                                  rotary=None if rope is None else (rope, width))
+        with monkeypatch.context() as mp:
+            mp.setattr(torch.Tensor, "new_empty", no_scratch)
+            outs.append(op(X, Wt, epilogue))
+        assert all(torch.equal(outs[0], o) for o in outs[1:])
+        a = xn if norm else x
+        want = O.linear(a, w, bias=b, gelu=bool(gelu), rope=table if tokens else None, tokens=tokens,
+                        width=width if tokens else 0, residual=None if residual is None else r)
+        check("without scratch", outs[0].cpu().numpy(), want,
+              bound(a, w, 1.42 if tokens else 1.13 if gelu else 1.0) + 1e-6)
