@@ -47,8 +47,9 @@ def _rows(t: torch.Tensor) -> tuple[torch.Tensor, int]:
     if t.dtype != torch.float32:
         raise ValueError("fused ops take float32 tensors")
     g, tok = t.shape[0], t.shape[1]
-    if t.is_contiguous():
-        # Dense as it is; callers use only its address and this stride.
+    if t.is_contiguous() and t.numel():
+        # Dense as it is; callers use only its address and this stride. (A call without elements is
+        # refused below: its row length is ambiguous.)
         return t, t.shape[2] * t.shape[3] if t.dim() == 4 else t.shape[2]
     try:
         flat = t.view(g, tok, -1)
@@ -207,7 +208,7 @@ def unit_norm(x: torch.Tensor, scale: Optional[torch.Tensor] = None) -> torch.Te
     require_optional(scale, "scale", x.device, (dim,))
     if not _usable():
         raise RuntimeError("the gfx950 kernels cannot run on this device")
-    flat = x if x.dim() == 2 else x.reshape(-1, dim)
+    flat = x if x.dim() == 2 and dim else x.reshape(-1, dim)
     if flat.stride(1) != 1:
         flat = flat.contiguous()
     out = x.new_empty(x.shape)

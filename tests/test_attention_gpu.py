@@ -341,3 +341,17 @@ def test_time_attention_is_repeatable(gpu, tokens):
     for i, out in enumerate(outs):
         check(f"repeat {i} T={tokens}", out.cpu().numpy(), expected)
     assert all(torch.equal(outs[0], o) for o in outs[1:]), "attention must be deterministic"
+
+
+def test_calls_without_elements_are_refused(gpu):
+    """Attention over no sequences or no tokens and a norm over no channels raise, as a row of unknown
+    length cannot be viewed; a norm of no rows is an empty result."""
+    for groups, tokens in ((0, 5), (3, 0)):
+        q = torch.empty((groups, tokens, 2, 64), device=gpu)
+        with pytest.raises(RuntimeError):
+            fused.attention(q, q, q)
+        with pytest.raises(RuntimeError):
+            fused.gated_attention(torch.empty((groups, tokens, 512), device=gpu), 2)
+    with pytest.raises(RuntimeError):
+        fused.unit_norm(torch.empty((3, 0), device=gpu))
+    assert tuple(fused.unit_norm(torch.empty((0, 64), device=gpu)).shape) == (0, 64)

@@ -104,6 +104,34 @@ def test_istft_frame_groups_and_unaligned_spectrum(gpu, frames, hop, offset):
                 1e-5 * np.abs(want).max())
 
 
+def test_istft_past_32_bit_sample_indices(gpu):
+    """2^31 samples a channel, where the overlap-add indexes in 64 bits: silence but for the first and
+    last frames, whose samples equal those of a clip of these frames alone (the oracle's, by the tests
+    above), bit for bit."""
+    hop, few = 1024, 12
+    frames = (1 << 31) // hop + 1
+    need = frames * (2 * 16400 + 16384) + (8 << 31)
+    if torch.cuda.mem_get_info(gpu)[0] < need + (16 << 30):
+        pytest.skip(f"needs {need >> 30} GiB of GPU memory")
+    spec = torch.from_numpy(W.normal((few, 1025, 2, 2), 48, 1.0)).to(gpu)
+    masks = torch.from_numpy(W.normal((2050, 2, few), 49, 1.0)).to(gpu)
+    want = S.istft(spec, masks, hop, (few - 1) * hop)
+    torch.cuda.empty_cache()
+    long_spec = torch.zeros((frames, 1025, 2, 2), device=gpu)
+    long_masks = torch.zeros((2050, 2, frames), device=gpu)
+    for part in (slice(0, few), slice(frames - few, frames)):
+        long_spec[part] = spec
+        long_masks[:, :, part] = masks
+    got = S.istft(long_spec, long_masks, hop, (frames - 1) * hop)
+    del long_spec, long_masks
+    tail = (few - 2) * hop
+    assert torch.equal(got[:, :tail], want[:, :tail])
+    assert torch.equal(got[:, -tail:], want[:, -tail:])
+    assert not got[:, few * hop + 1024:1 << 20].any() and not got[:, 1 << 30:(1 << 30) + (1 << 20)].any()
+    del got
+    torch.cuda.empty_cache()
+
+
 @pytest.mark.parametrize("depth", [1, 3])
 def test_forward_matches_oracle_tiny(gpu, depth):
     """Two stems, three overlapping bands, 101 frames (time kernel), 3 bands (band kernel).
