@@ -7,9 +7,11 @@
 // logits, 3 width + width / 64 of them, rounded up to a 32-column block; the packed layout's
 // zero padding after them is never read by the attention kernels and is left as it is.
 //
-// 128 rows per workgroup (96 at dim 512): their fp16 operand rows sit in LDS for the whole block
-// as B fragments of v_mfma_f32_32x32x16_f16 (straight from HBM with direct-to-LDS loads), with the
-// rows' rotary cos / sin (32 + 32 per row) next to them. The 8 waves walk the output in pairs of
+// 128 rows per workgroup (96 at dim 512; a 32-row tile less where that still is one round): their
+// fp16 operand rows sit in LDS for the whole block as they lie in memory (direct-to-LDS loads of a
+// contiguous kilobyte, 16-byte chunks XOR-swizzled by row), where a v_mfma_f32_32x32x16_f16 B fragment
+// is one 16-byte read per lane, with the rows' rotary cos / sin (32 + 32 per row) next to them. Few row
+// blocks split their columns over up to six workgroups. The 8 waves walk the output in pairs of
 // 32-column blocks (pair p on SIMD p % 4, so the SIMDs get the same count); per pair a wave
 // accumulates all its rows (4 or 3 32-row MFMA tiles per block) over K, so each operand B
 // fragment read from LDS feeds two MFMAs and each weight A fragment (a contiguous kilobyte of the
@@ -49,7 +51,7 @@ __device__ __forceinline__ void store_gap() {
   __builtin_amdgcn_sched_barrier(0);
 }
 
-// SD = dim / 16 k steps (dims 128 - 512); NR 32-row tiles per row block (4; 3 at dim 512).
+// SD = dim / 16 k steps (dims 128 - 512); NR 32-row tiles per row block (4; 3 at dim 512; or one less).
 // TANH: the mask heads' hidden layer (bias + tanh on every column, no rotary table, p.batch
 // products of p.rows rows each).
 template <int SD, int NR, bool TANH = false>

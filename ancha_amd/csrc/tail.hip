@@ -1,5 +1,5 @@
-// Fused tail of the RoFormer block on gfx950: everything after the attention core, 64 rows at
-// a time, with the feed-forward hidden activation kept on chip (crates/ancha-models/src/
+// Fused tail of the RoFormer block on gfx950: everything after the attention core, 32 to 96
+// rows at a time, with the feed-forward hidden activation kept on chip (crates/ancha-models/src/
 // roformer.rs:487-519, Transformer::forward_kernels after its gated_attention call):
 //   x1 = x + attended . W_out                          out projection + residual
 //   h  = fp16(GELU(fp16(unit_norm(x1)) . W1' + b1))    FF in (sqrt(dim)*gamma folded into W1')
@@ -13,7 +13,7 @@
 // features x 16 k) come from the weights, stored at block load in a fragment-major layout (one
 // 1 KB fragment per (32-feature block, 16-k step), lane-ordered, so a wave's A load is one
 // contiguous kilobyte); B fragments (16 k x 32 rows) come from LDS in the same fragment-major
-// order. Lane l holds D rows (features) 8q + 4(l/32) + e (q, e < 4) of row l % 32. A lane's 8
+// order, or for the out projection from the attended rows as they lie in memory. Lane l holds D rows (features) 8q + 4(l/32) + e (q, e < 4) of row l % 32. A lane's 8
 // values of one 16-feature step are thus features {4h..4h+3, 8+4h..8+4h+3} (h = l/32): written
 // as fp16 they are directly lane l's B fragment of the next product if the next product's
 // weights take their k (= feature) axis in that order, i.e. permuted within each 16-block by
@@ -32,10 +32,10 @@
 //
 // Workgroup: 32 NJ rows (64; 32 or 96 in smaller calls), 4 waves, one per feature quarter (and
 // SIMD); two workgroups per CU, whose phases drift apart, so one's GELU / norm VALU work runs beside
-// the other's MFMAs. The out accumulator (rows x dim) stays in registers from the residual load to the final store; the
-// hidden dimension runs in chunks of 256 units up to dim 384, 128 at dim 512 (per chunk: FF-in
-// for 64 or 32 hidden units per wave, GELU, the chunk's fp16 activation to LDS, then its FF-out
-// contribution).
+// the other's MFMAs (96 rows: one workgroup and one wave per SIMD). The out accumulator (rows x dim)
+// stays in registers from the residual load to the final store; the hidden dimension runs in chunks of
+// 256 units up to dim 384, 128 at dim 512 (per chunk: FF-in for 64 or 32 hidden units per wave, GELU,
+// the chunk's fp16 activation to LDS, then its FF-out contribution).
 #include "buffer.hpp"
 #include "common.hpp"
 #include "gemm.hpp"
@@ -59,7 +59,7 @@ __device__ __forceinline__ u32x4 pack_frag(const f32x16& d, int sub, float s) {
                pack_h2(d[o + 4] * s, d[o + 5] * s), pack_h2(d[o + 6] * s, d[o + 7] * s)};
 }
 
-// Sum over the 4 feature-quarter waves of per-row partials (red: [4][128] floats in LDS).
+// Sum over the 4 feature-quarter waves of per-row partials (red: [4][32 NJ] floats in LDS).
 // Every wave calls it; it ends with the totals of this lane's rows in tot[].
 template <int NJ>
 __device__ __forceinline__ void row_totals(float* red, const float (&part)[NJ], float (&tot)[NJ],
@@ -100,7 +100,7 @@ __global__ __launch_bounds__(kWaves * 64, NJ > 2 ? 1 : 2) void block_tail_kernel
   __shared__ __attribute__((aligned(16))) unsigned char lds[kLds];
   unsigned char* const X = lds;         // xh1: fragment (jb, s) at (jb * SD + s) * 1 KB
   unsigned char* const H = lds + kX;    // hidden chunk: fragment (jb, s) at (jb * kSC + s) * 1 KB
-  float* const red = reinterpret_cast<float*>(H);  // [4][128] row partials (aliases H)
+  float* const red = reinterpret_cast<float*>(H);  // [4][32 NJ] row partials (aliases H)
 
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);

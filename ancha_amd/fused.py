@@ -194,7 +194,7 @@ def linear(x: torch.Tensor, weight: torch.Tensor,
 
 def norm_linear(x: torch.Tensor, weight: torch.Tensor,
                 epilogue: Optional[Epilogue] = None) -> Optional[torch.Tensor]:
-    """``linear(unit_norm(x), weight, epilogue)`` in one kernel (the row norm scales the
+    """``linear(unit_norm(x), weight, epilogue)`` in one call (the row norm scales the
     product), the call pattern of Transformer::forward_kernels (roformer.rs:477-485, :497-505)."""
     return _linear(x, weight, epilogue or Epilogue(), norm=True)
 
